@@ -359,13 +359,8 @@ static void axis_eigen(int n, double c, bool periodic, std::vector<double> &Q,
 // right-hand side and result of one V-cycle on level 0 (natural-order vectors)
 template <typename T> static void mg_bind_level0(MGLevelT<T> &L0, const T *rhs, T *out)
 {
-    if (L0.split) {
-        L0.fin = rhs;
-        L0.uout = out;
-    } else {
-        L0.f = const_cast<T *>(rhs);
-        L0.u = out;
-    }
+    L0.f = const_cast<T *>(rhs);
+    L0.u = out;
 }
 
 // one V-cycle on rhs -> out (natural-order level-0 vectors).  With cfg.mg_graphs the
@@ -444,13 +439,7 @@ template <typename T> static int setup_multigrid(cfdmx_ctx *ctx)
     L.fx = L.fy = L.fz = 1;
     L.zper = g.zper;
     divs(L);
-    // a level with even nz is stored by colour; level 0 then has u and f of its own,
-    // filled from and returned to the natural-order Krylov vectors
-    L.split = L.nz % 2 == 0;
-    if (L.split) {
-        ALLOC(L.u, N);
-        ALLOC(L.f, N);
-    }
+    if (L.nz % 2 == 0) ALLOC(L.ub, N / 2);
     lev.push_back(L);
     for (;;) {
         const MGLevelT<T> &P = lev.back();
@@ -477,7 +466,7 @@ template <typename T> static int setup_multigrid(cfdmx_ctx *ctx)
         C.fz = fz;
         C.zper = g.zper;
         divs(C);
-        C.split = C.nz % 2 == 0;
+        if (C.nz % 2 == 0) ALLOC(C.ub, (size_t)C.n / 2);
         ALLOC(C.u, (size_t)C.n);
         ALLOC(C.f, (size_t)C.n);
         lev.push_back(C);
@@ -489,9 +478,7 @@ template <typename T> static int setup_multigrid(cfdmx_ctx *ctx)
                             "coarse solve takes at most %d cells and %d per axis); use sizes "
                             "with more factors of two",
              g.nxc, g.nyc, g.nzc, B.nx, B.ny, B.nz, kMGCoarseCells, kMGCoarseAxis);
-    // the coarsest level is solved in natural order (a single level is then bound to the
-    // Krylov vectors directly); its operator is the Kronecker sum of three 1-D chains
-    B.split = 0;
+    // the coarsest level's operator is the Kronecker sum of three 1-D chains
     {
         std::vector<double> Qx, Qy, Qz, lx, ly, lz;
         axis_eigen(B.nx, (double)B.cx, false, Qx, lx);
@@ -505,6 +492,7 @@ template <typename T> static int setup_multigrid(cfdmx_ctx *ctx)
         HIPCHK(hipMemcpy(dm, pack.data(), pack.size() * sizeof(T), hipMemcpyHostToDevice));
         B.fd = dm;
     }
+    mg_plan(lev.data(), (int)lev.size());
     ALLOC(ctx->pbs, 1);
     ALLOC(ctx->pb_part, 2 * (size_t)g.nblocks + 64);
     ALLOC(ctx->mix, 4);

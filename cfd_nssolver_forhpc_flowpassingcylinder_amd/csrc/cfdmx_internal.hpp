@@ -95,16 +95,15 @@ struct MGLevelT {
     int fx, fy, fz;     // coarsening factors from the finer level (1 or 2)
     int zper;
     FastDiv dz, dy, dzh; // divisions by nz, ny and nz/2
-    // u and f of the level.  split = 1 (levels with even nz): stored by colour, the red
-    // cells ((i + j + k) even) in [0, n/2) and the black ones in [n/2, n), cell k of row
-    // (i, j) at (i*ny + j)*(nz/2) + k/2 of its colour's half.  split = 0: natural order.
-    T *u, *f;
-    int split;
-    // level 0 when split: the natural-order right-hand side and result vectors of the
-    // Krylov solve (read by the first sweep, written by the last)
-    const T *fin;
-    T *uout;
-    // coarsest level (stored in natural order): the orthonormal eigenvectors of the 1-D
+    // u and f of the level, natural order; on level 0 the result and right-hand side
+    // vectors of the Krylov solve.  ub: the black cells of u between the two halves of a
+    // cycle (levels that sweep in one pass: see cfdmx_mg_sweep.hpp), pair kk of row (i, j)
+    // at (i*ny + j)*(nz/2) + kk
+    T *u, *f, *ub;
+    // tiling of the one-pass kernels (mg_plan): pairs a thread, rows, pairs and planes a block;
+    // sp = 0: a launch per half sweep
+    int sp, sty, stz, scx;
+    // coarsest level: the orthonormal eigenvectors of the 1-D
     // operators, Qx (nx x nx, row m = mode m), Qy, Qz, then their eigenvalues (nx, ny, nz
     // values); the level's operator is their Kronecker sum
     const T *fd;
@@ -113,15 +112,37 @@ struct MGLevelT {
 // the hierarchy stops at the first level of at most this many cells, solved exactly
 constexpr int kMGCoarseCells = 512;
 constexpr int kMGCoarseAxis = 512; // largest axis length of that level
-// a level above the coarsest of at most this many cells (stored by colour) runs its whole
-// V-cycle, the coarse solve included, in one workgroup with its u in LDS (k_mg_tail)
-constexpr int kMGTailCells = 4096;
+// the first level of at most this many cells and all below it run in one workgroup, in LDS
+// (k_mg_tail).  A level with even nz in two one-pass launches takes 14 us at 64x32x2, level
+// with the workgroup's 13 us in float and ahead of its 20 us in double (V-cycles 173 against
+// 177 us and 238 against 252 us at 512x256x64); one with odd nz would take a launch per half
+// sweep, where the workgroup wins up to twice the size (55 against 70 us at 96x48x6)
+constexpr int kMGTailCells = 2048, kMGTailCellsOdd = 4096;
+constexpr int kMGTailLevels = 8;
+
+constexpr size_t kMGSweepLds = 160 * 1024; // LDS of a CU, which one block may take
+// rows of more pairs than this may be cut into parts (shorter ones are always whole)
+constexpr int kMGLongRow = 48;
+// one level's half V-cycle in one pass (cfdmx_mg_sweep.hpp)
+template <typename T>
+struct MGSweepT {
+    int nx, ny, nz, half;          // level sizes, half = nz / 2
+    int fx, fy, fz, cny, cnz;      // coarsening factors and the coarse level's ny, nz
+    int ty, rows, tpr, cxl;        // rows owned, rows held (ty + 8), threads a row, planes
+    int tz, pairs;                 // pairs of a row owned (half: whole rows) and held
+    int njt, nkt, nblk;            // tiles in y and z, blocks
+    T cx, cy, cz;
+    const T *f, *e;                // right-hand side; coarse correction (up)
+    T *ub, *fc, *u;                // black half; coarse right-hand side (down); result (up)
+};
 
 struct PBState {
     double rho, alpha, omega, beta, norm0, res, tol;
     int iter, maxit, done;
 };
 
+template <typename T>
+void mg_plan(MGLevelT<T> *L, int nlev);
 template <typename T>
 void launch_mg_vcycle(hipStream_t s, const MGLevelT<T> *L, int nlev, int l);
 template <typename T>

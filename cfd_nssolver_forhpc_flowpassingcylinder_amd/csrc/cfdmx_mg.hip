@@ -13,19 +13,17 @@
 // exactly by fast diagonalisation (the 1-D eigenbases of its three axes, computed on the
 // host).  Every inner product accumulates in double.
 //
-// A level with even nz stores u and f by colour (red cells, then black cells), and its
-// kernels take one thread per z-pair (cells 2kk and 2kk+1 of an (i, j) row), so a half
-// sweep runs one thread per cell of its colour and touches only the values it uses:
-//   first sweep from u = 0 (red u = f/d, then black from the red values) -- one kernel;
-//     on level 0 it also stores the natural-order right-hand side by colour;
-//   half sweeps; on level 0 the last one writes the result in natural order;
-//   restriction (one thread per coarse cell);
-//   prolongation fused with the next red half sweep: the red cell reads its black
-//   neighbours corrected on the fly; the black cells are left uncorrected, since the
-//   black half sweep that follows overwrites them without reading them.
-// Levels with odd nz are stored in natural order and use one thread per cell.  The
-// arithmetic of every cell update (terms, weights, order) is the same in either layout.
+// Every level is stored in natural order.  A level with even nz takes two kernels a cycle,
+// one on the way down and one on the way up, each passing over the level once with all its
+// half sweeps (cfdmx_mg_sweep.hpp).  The smallest levels run in one workgroup, in LDS.
+// Levels with odd nz above those take a launch per half sweep, one thread per cell.  The
+// arithmetic of every cell update (terms, weights, order) is the same in each form.
+//
+// Measured, a V-cycle before (a launch per half sweep, colours stored apart) and after:
+// 350 -> 173 us in float and 508 -> 238 us in double at 512x256x64, 2.4 ms -> 660 us in
+// float at 1024x512x128.
 #include "cfdmx_internal.hpp"
+#include "cfdmx_mg_sweep.hpp"
 
 namespace cfdmx {
 
@@ -38,18 +36,6 @@ __device__ __forceinline__ void mg_coords(const MGLevelT<T> &L, int n, int &i, i
     k = n - (int)t * L.nz;
     i = (int)fdiv(t, L.dy);
     j = (int)t - i * L.ny;
-}
-
-// z-pair m of a level with even nz: row (i, j) and the pair's first cell 2kk
-template <typename T>
-__device__ __forceinline__ void mg_pair(const MGLevelT<T> &L, int m, int &i, int &j, int &k0,
-                                        int &row)
-{
-    const int half = L.nz >> 1;
-    row = (int)fdiv((unsigned)m, L.dzh);
-    k0 = 2 * (m - row * half);
-    i = (int)fdiv((unsigned)row, L.dy);
-    j = row - i * L.ny;
 }
 
 template <typename T>
@@ -95,306 +81,7 @@ __device__ __forceinline__ T mg_nbsum(const MGLevelT<T> &L, int n, int i, int j,
     return s;
 }
 
-// storage index of cell (i, j, k) of a level (natural or by colour, see MGLevelT)
-template <typename T>
-__device__ __forceinline__ int mg_at(const MGLevelT<T> &L, int i, int j, int k)
-{
-    const int row = i * L.ny + j;
-    if (!L.split) return row * L.nz + k;
-    return ((i + j + k) & 1) * (L.n >> 1) + row * (L.nz >> 1) + (k >> 1);
-}
-
-// mg_nbsum by coordinates: v(a, b, c) gives the value of cell (a, b, c); the same
-// terms, weights and order, and the cell itself with weight 0 for a missing neighbour
-template <typename T, class V>
-__device__ __forceinline__ T mg_nbsum_c(const MGLevelT<T> &L, int i, int j, int k, V &&v)
-{
-    const bool xm = i > 0, xp = i < L.nx - 1, ym = j > 0, yp = j < L.ny - 1;
-    T s = (T)0;
-    s += (xm ? L.cx : (T)0) * v(xm ? i - 1 : i, j, k);
-    s += (xp ? L.cx : (T)0) * v(xp ? i + 1 : i, j, k);
-    s += (ym ? L.cy : (T)0) * v(i, ym ? j - 1 : j, k);
-    s += (yp ? L.cy : (T)0) * v(i, yp ? j + 1 : j, k);
-    if (L.nz > 1) {
-        const bool zm = L.zper || k > 0, zp = L.zper || k < L.nz - 1;
-        const int km = k > 0 ? k - 1 : (zm ? L.nz - 1 : k);
-        const int kp = k < L.nz - 1 ? k + 1 : (zp ? 0 : k);
-        s += (zm ? L.cz : (T)0) * v(i, j, km);
-        s += (zp ? L.cz : (T)0) * v(i, j, kp);
-    }
-    return s;
-}
-
-// ---- levels with even nz: stored by colour, one thread per z-pair ----
-// Thread m is the z-pair (2kk, 2kk+1) of row (i, j); its cell of colour c is
-// k = 2kk + ((i + j + c) & 1), at c*n/2 + m.  The neighbours of that cell are the
-// other colour's cells at the same kk of the rows (i +- 1, j) and (i, j +- 1), and at
-// kk - 1 + p and kk + p of its own row (p = (i + j + c) & 1; periodic z wraps kk).  A
-// half sweep so reads the other colour's half and its own colour's f, and writes its
-// own colour's half: whole cache lines of the values it uses.
-
-// half sweep over colour c: the sum of mg_nbsum (same terms and order; a missing
-// neighbour reads the cell itself with weight 0)
-template <typename T>
-__device__ __forceinline__ T mg_split_update(const MGLevelT<T> &L, const T *u, int m, int row,
-                                             int i, int j, int kk, int c, int &own, int &k)
-{
-    const int half = L.nz >> 1, hn = L.n >> 1;
-    const int pc = (i + j + c) & 1;
-    k = 2 * kk + pc;
-    own = c * hn + m;
-    const int ob = (1 - c) * hn;
-    const int sxh = L.ny * half;
-    const bool xm = i > 0, xp = i < L.nx - 1, ym = j > 0, yp = j < L.ny - 1;
-    T s = (T)0;
-    s += (xm ? L.cx : (T)0) * u[xm ? ob + m - sxh : own];
-    s += (xp ? L.cx : (T)0) * u[xp ? ob + m + sxh : own];
-    s += (ym ? L.cy : (T)0) * u[ym ? ob + m - half : own];
-    s += (yp ? L.cy : (T)0) * u[yp ? ob + m + half : own];
-    // nz is even, so nz > 1
-    const bool zm = L.zper || k > 0, zp = L.zper || k < L.nz - 1;
-    const int kkm = (k > 0) ? kk - 1 + pc : half - 1;  // k - 1, or nz - 1 wrapped
-    const int kkp = (k < L.nz - 1) ? kk + pc : 0;      // k + 1, or 0 wrapped
-    s += (zm ? L.cz : (T)0) * u[zm ? ob + row * half + kkm : own];
-    s += (zp ? L.cz : (T)0) * u[zp ? ob + row * half + kkp : own];
-    return s;
-}
-
-// the half sweep of colour c at z-pair m (the kernels below and the tail kernel)
-template <typename T>
-__device__ __forceinline__ void mg_smooth_at(const MGLevelT<T> &L, int m, int colour)
-{
-    int i, j, k0, row;
-    mg_pair(L, m, i, j, k0, row);
-    int own, k;
-    const T s = mg_split_update(L, L.u, m, row, i, j, k0 >> 1, colour, own, k);
-    L.u[own] = (L.f[own] + s) / mg_diag(L, i, j, k);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_mg_smooth(MGLevelT<T> L, int colour)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= (L.n >> 1)) return;
-    mg_smooth_at(L, m, colour);
-}
-
-// The same half sweep with two neighbouring cells of a colour per thread (FP64 levels
-// with nz a multiple of 4, so a row holds whole pairs and a pair's first index is even):
-// their f, the x and y neighbours of both and the other colour's pair beside them move as
-// one 16-byte vector each, and the z neighbours take one more value.  Each cell's terms,
-// weights and order are mg_split_update's, and an absent neighbour reads the cell itself
-// with weight 0, as there, so the result is the same.
-template <typename T> struct Pair;
-template <> struct Pair<double> {
-    using V = double2;
-};
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_mg_smooth2(MGLevelT<T> L, int colour)
-{
-    using V = typename Pair<T>::V;
-    const int m = 2 * (blockIdx.x * blockDim.x + threadIdx.x);
-    const int half = L.nz >> 1, hn = L.n >> 1;
-    if (m >= hn) return;
-    int i, j, k0, row;
-    mg_pair(L, m, i, j, k0, row);
-    const int kk = k0 >> 1; // even: the pair is (kk, kk + 1)
-    const int pc = (i + j + colour) & 1;
-    const int own = colour * hn + m, ob = (1 - colour) * hn;
-    const int sxh = L.ny * half;
-    const bool xm = i > 0, xp = i < L.nx - 1, ym = j > 0, yp = j < L.ny - 1;
-    const T *u = L.u;
-    const V vxm = *reinterpret_cast<const V *>(u + (xm ? ob + m - sxh : own));
-    const V vxp = *reinterpret_cast<const V *>(u + (xp ? ob + m + sxh : own));
-    const V vym = *reinterpret_cast<const V *>(u + (ym ? ob + m - half : own));
-    const V vyp = *reinterpret_cast<const V *>(u + (yp ? ob + m + half : own));
-    const V oz = *reinterpret_cast<const V *>(u + ob + m);
-    const V fv = *reinterpret_cast<const V *>(L.f + own);
-    // z neighbours (cells A = kk and B = kk + 1 at k = 2 kk + pc and k + 2): with pc = 0,
-    // A's -z is the other colour at kk - 1 (wrapped to half - 1 at k = 0) and the rest are
-    // the pair beside; with pc = 1, B's +z is the other colour at kk + 2 (wrapped to 0 at
-    // k = nz - 1)
-    const int kA = 2 * kk + pc, kB = kA + 2;
-    T zmA, zpA, zmB, zpB;
-    bool hzmA = true, hzpB = true;
-    if (pc == 0) {
-        hzmA = L.zper || kA > 0;
-        zmA = u[hzmA ? (kA > 0 ? ob + m - 1 : ob + row * half + half - 1) : own];
-        zpA = oz.x;
-        zmB = oz.x;
-        zpB = oz.y;
-    } else {
-        zmA = oz.x;
-        zpA = oz.y;
-        zmB = oz.y;
-        hzpB = L.zper || kB < L.nz - 1;
-        zpB = u[hzpB ? (kB < L.nz - 1 ? ob + m + 2 : ob + row * half) : own + 1];
-    }
-    const T wx = L.cx, wy = L.cy, wz = L.cz, z0 = (T)0;
-    T sA = (T)0, sB = (T)0;
-    sA += (xm ? wx : z0) * vxm.x;
-    sB += (xm ? wx : z0) * vxm.y;
-    sA += (xp ? wx : z0) * vxp.x;
-    sB += (xp ? wx : z0) * vxp.y;
-    sA += (ym ? wy : z0) * vym.x;
-    sB += (ym ? wy : z0) * vym.y;
-    sA += (yp ? wy : z0) * vyp.x;
-    sB += (yp ? wy : z0) * vyp.y;
-    sA += (hzmA ? wz : z0) * zmA;
-    sB += wz * zmB;
-    sA += wz * zpA;
-    sB += (hzpB ? wz : z0) * zpB;
-    V out;
-    out.x = (fv.x + sA) / mg_diag(L, i, j, kA);
-    out.y = (fv.y + sB) / mg_diag(L, i, j, kB);
-    *reinterpret_cast<V *>(L.u + own) = out;
-}
-
-// the last half sweep of level 0 (black), writing the result of both colours to the
-// natural-order output vector
-template <typename T>
-__global__ void __launch_bounds__(256) k_mg_smooth_out(MGLevelT<T> L)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= (L.n >> 1)) return;
-    int i, j, k0, row;
-    mg_pair(L, m, i, j, k0, row);
-    int own, k;
-    const T s = mg_split_update(L, L.u, m, row, i, j, k0 >> 1, 1, own, k);
-    const T ub = (L.f[own] + s) / mg_diag(L, i, j, k);
-    const int kr = k0 + ((i + j) & 1);
-    L.uout[row * L.nz + k] = ub;
-    L.uout[row * L.nz + kr] = L.u[m];
-}
-
-// first sweep from u = 0: red u = f/d, then black u = (f + sum c (f/d)(red nb)) / d.
-// On level 0 f comes in natural order (fin) and is stored by colour here.
-template <typename T>
-__device__ __forceinline__ void mg_smooth_first_at(const MGLevelT<T> &L, int m)
-{
-    int i, j, k0, row;
-    mg_pair(L, m, i, j, k0, row);
-    const int hn = L.n >> 1;
-    const int kr = k0 + ((i + j) & 1), kb = k0 + ((i + j + 1) & 1);
-    T fr, fb;
-    if (L.fin) {
-        fr = L.fin[row * L.nz + kr];
-        fb = L.fin[row * L.nz + kb];
-        L.f[m] = fr;
-        L.f[hn + m] = fb;
-    } else {
-        fr = L.f[m];
-        fb = L.f[hn + m];
-    }
-    L.u[m] = fr / mg_diag(L, i, j, kr);
-    const T *fin = L.fin, *f = L.f;
-    const T s = mg_nbsum_c(L, i, j, kb, [&](int a, int b, int c) {
-        const T fv = fin ? fin[(a * L.ny + b) * L.nz + c] : f[mg_at(L, a, b, c)];
-        return fv / mg_diag(L, a, b, c);
-    });
-    L.u[hn + m] = (fb + s) / mg_diag(L, i, j, kb);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_mg_smooth_first(MGLevelT<T> L)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= (L.n >> 1)) return;
-    mg_smooth_first_at(L, m);
-}
-
-// prolongation fused with the red half sweep (see the file comment)
-template <typename T>
-__device__ __forceinline__ void mg_prolong_smooth_at(const MGLevelT<T> &F, const MGLevelT<T> &C,
-                                                     int m)
-{
-    int i, j, k0, row;
-    mg_pair(F, m, i, j, k0, row);
-    const int k = k0 + ((i + j) & 1);
-    const int shx = C.fx >> 1, shy = C.fy >> 1, shz = C.fz >> 1;
-    const T *u = F.u, *e = C.u;
-    const T s = mg_nbsum_c(F, i, j, k, [&](int a, int b, int c) {
-        return u[mg_at(F, a, b, c)] + e[mg_at(C, a >> shx, b >> shy, c >> shz)];
-    });
-    F.u[m] = (F.f[m] + s) / mg_diag(F, i, j, k);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_mg_prolong_smooth(MGLevelT<T> F, MGLevelT<T> C)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= (F.n >> 1)) return;
-    mg_prolong_smooth_at(F, C, m);
-}
-
-// ---- z-only coarsening (fx = fy = 1, fz = 2) of a level stored by colour: the
-// children of coarse cell (i, j, kk) are fine z-pair m, so these run one thread per
-// z-pair with the fast neighbour indexing ----
-
-// coarse right-hand side: the mean of the two children's residuals f - A u (the same
-// expression and order as k_mg_restrict)
-template <typename T>
-__global__ void __launch_bounds__(256) k_mg_restrict_z(MGLevelT<T> F, MGLevelT<T> C)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= (F.n >> 1)) return;
-    int i, j, k0, row;
-    mg_pair(F, m, i, j, k0, row);
-    const int kk = k0 >> 1;
-    T r[2];
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        int own, k;
-        const T s = mg_split_update(F, F.u, m, row, i, j, kk, c, own, k);
-        r[c] = F.f[own] - (mg_diag(F, i, j, k) * F.u[own] - s);
-    }
-    // children in z order: cell 2kk has colour (i + j) & 1
-    const bool even_red = ((i + j) & 1) == 0;
-    T acc = (T)0;
-    acc += even_red ? r[0] : r[1];
-    acc += even_red ? r[1] : r[0];
-    C.f[mg_at(C, i, j, kk)] = acc / (T)2;
-}
-
-// prolongation fused with the red half sweep: each black neighbour is corrected by its
-// parent's value, the parent of fine cell (a, b, c) being coarse cell (a, b, c/2)
-template <typename T>
-__global__ void __launch_bounds__(256) k_mg_prolong_smooth_z(MGLevelT<T> F, MGLevelT<T> C)
-{
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= (F.n >> 1)) return;
-    int i, j, k0, row;
-    mg_pair(F, m, i, j, k0, row);
-    const int kk = k0 >> 1;
-    const int half = F.nz >> 1, hn = F.n >> 1, sxh = F.ny * half;
-    const int pr = (i + j) & 1;
-    const int k = k0 + pr;
-    const T *u = F.u, *e = C.u;
-    // fine black index (other half) and coarse index of each neighbour, in the order of
-    // mg_nbsum; a missing neighbour is the red cell itself, weight 0
-    const bool xm = i > 0, xp = i < F.nx - 1, ym = j > 0, yp = j < F.ny - 1;
-    const bool zm = F.zper || k > 0, zp = F.zper || k < F.nz - 1;
-    const int kzm = k > 0 ? k - 1 : F.nz - 1, kzp = k < F.nz - 1 ? k + 1 : 0;
-    const int kkm = (k > 0) ? kk - 1 + pr : half - 1;
-    const int kkp = (k < F.nz - 1) ? kk + pr : 0;
-    // branch-free: the indices are selected, then both values are loaded unconditionally
-    auto val = [&](bool ok, int fine, int a, int b, int c) {
-        const int fi = ok ? hn + fine : m;
-        const int ci = mg_at(C, ok ? a : i, ok ? b : j, (ok ? c : k) >> 1);
-        return u[fi] + e[ci];
-    };
-    T s = (T)0;
-    s += (xm ? F.cx : (T)0) * val(xm, m - sxh, i - 1, j, k);
-    s += (xp ? F.cx : (T)0) * val(xp, m + sxh, i + 1, j, k);
-    s += (ym ? F.cy : (T)0) * val(ym, m - half, i, j - 1, k);
-    s += (yp ? F.cy : (T)0) * val(yp, m + half, i, j + 1, k);
-    s += (zm ? F.cz : (T)0) * val(zm, row * half + kkm, i, j, kzm);
-    s += (zp ? F.cz : (T)0) * val(zp, row * half + kkp, i, j, kzp);
-    F.u[m] = (F.f[m] + s) / mg_diag(F, i, j, k);
-}
-
-// ---- levels with odd nz: one thread per cell ----
+// ---- a launch per half sweep, one thread per cell ----
 
 // half sweep; zero_first: u starts at zero (the other colour is written 0).  With
 // periodic z and odd nz > 1 the planes k = 0 and k = nz-1 hold the same colour and are
@@ -420,13 +107,19 @@ __global__ void __launch_bounds__(256) k_mg_smooth_cell(MGLevelT<T> L, int colou
 }
 
 template <typename T>
+__device__ __forceinline__ void mg_prolong_at(const MGLevelT<T> &F, const MGLevelT<T> &C, int n)
+{
+    int i, j, k;
+    mg_coords(F, n, i, j, k);
+    F.u[n] += C.u[((i >> (C.fx >> 1)) * C.ny + (j >> (C.fy >> 1))) * C.nz + (k >> (C.fz >> 1))];
+}
+
+template <typename T>
 __global__ void __launch_bounds__(256) k_mg_prolong(MGLevelT<T> F, MGLevelT<T> C)
 {
     const int n = blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= F.n) return;
-    int i, j, k;
-    mg_coords(F, n, i, j, k);
-    F.u[n] += C.u[mg_at(C, i >> (C.fx >> 1), j >> (C.fy >> 1), k >> (C.fz >> 1))];
+    mg_prolong_at(F, C, n);
 }
 
 // coarse right-hand side: mean over the children of the fine residual f - A u
@@ -446,14 +139,12 @@ __device__ __forceinline__ void mg_restrict_at(const MGLevelT<T> &F, const MGLev
         const bool ok = a < C.fx && b < C.fy && c < C.fz;
         const int i = I * C.fx + (ok ? a : 0), j = J * C.fy + (ok ? b : 0),
                   k = K * C.fz + (ok ? c : 0);
-        const int n = mg_at(F, i, j, k);
-        const T s = mg_nbsum_c(F, i, j, k, [&](int x, int y, int z) {
-            return u[mg_at(F, x, y, z)];
-        });
+        const int n = (i * F.ny + j) * F.nz + k;
+        const T s = mg_nbsum(F, n, i, j, k, [&](int x, int, int, int) { return u[x]; });
         const T r = F.f[n] - (mg_diag(F, i, j, k) * u[n] - s);
         acc += ok ? r : (T)0;
     }
-    C.f[mg_at(C, I, J, K)] = acc / (T)(C.fx * C.fy * C.fz);
+    C.f[m] = acc / (T)(C.fx * C.fy * C.fz);
 }
 
 template <typename T>
@@ -471,11 +162,30 @@ __global__ void __launch_bounds__(256) k_mg_restrict(MGLevelT<T> F, MGLevelT<T> 
 // for the mean-free part of f.  One workgroup: the six 1-D transforms run through LDS,
 // a barrier apart.
 constexpr int kMGCoarseThreads = 1024;
+// sum over q < n of Q[q * sq] * a[q * sa], in order; the loads of eight terms overlap
 template <typename T>
-__device__ __forceinline__ void mg_coarse_solve(const MGLevelT<T> &L, T *a, T *b)
+__device__ __forceinline__ T mg_dot(const T *Q, int sq, const T *a, int sa, int n)
+{
+    T acc = (T)0;
+    int q = 0;
+    for (; q + 8 <= n; q += 8) {
+        T x[8], y[8];
+#pragma unroll
+        for (int w = 0; w < 8; ++w) x[w] = Q[(q + w) * sq], y[w] = a[(q + w) * sa];
+#pragma unroll
+        for (int w = 0; w < 8; ++w) acc += x[w] * y[w];
+    }
+    for (; q < n; ++q) acc += Q[q * sq] * a[q * sa];
+    return acc;
+}
+
+// Qx: the eigenvectors and eigenvalues (MGLevelT::fd or its copy in LDS); L.f may be b, and
+// L.u is written last, from b
+template <typename T>
+__device__ __forceinline__ void mg_coarse_solve(const MGLevelT<T> &L, const T *Qx, T *a, T *b)
 {
     const int nx = L.nx, ny = L.ny, nz = L.nz;
-    const T *Qx = L.fd, *Qy = Qx + nx * nx, *Qz = Qy + ny * ny;
+    const T *Qy = Qx + nx * nx, *Qz = Qy + ny * ny;
     const T *lx = Qz + nz * nz, *ly = lx + nx, *lz = ly + ny;
     const int tid = threadIdx.x, nt = blockDim.x;
     for (int n = tid; n < L.n; n += nt) a[n] = L.f[n];
@@ -484,24 +194,19 @@ __device__ __forceinline__ void mg_coarse_solve(const MGLevelT<T> &L, T *a, T *b
     for (int n = tid; n < L.n; n += nt) {
         int m, j, k;
         mg_coords(L, n, m, j, k);
-        T acc = (T)0;
-        for (int i = 0; i < nx; ++i) acc += Qx[m * nx + i] * a[(i * ny + j) * nz + k];
-        b[n] = acc;
+        b[n] = mg_dot(Qx + m * nx, 1, a + j * nz + k, ny * nz, nx);
     }
     __syncthreads();
     for (int n = tid; n < L.n; n += nt) {
         int mx, m, k;
         mg_coords(L, n, mx, m, k);
-        T acc = (T)0;
-        for (int j = 0; j < ny; ++j) acc += Qy[m * ny + j] * b[(mx * ny + j) * nz + k];
-        a[n] = acc;
+        a[n] = mg_dot(Qy + m * ny, 1, b + mx * ny * nz + k, nz, ny);
     }
     __syncthreads();
     for (int n = tid; n < L.n; n += nt) {
         int mx, my, m;
         mg_coords(L, n, mx, my, m);
-        T acc = (T)0;
-        for (int k = 0; k < nz; ++k) acc += Qz[m * nz + k] * a[(mx * ny + my) * nz + k];
+        const T acc = mg_dot(Qz + m * nz, 1, a + (mx * ny + my) * nz, 1, nz);
         const T lam = lx[mx] + ly[my] + lz[m];
         b[n] = (mx == 0 && my == 0 && m == 0) ? (T)0 : acc / lam;
     }
@@ -510,90 +215,129 @@ __device__ __forceinline__ void mg_coarse_solve(const MGLevelT<T> &L, T *a, T *b
     for (int n = tid; n < L.n; n += nt) {
         int mx, my, k;
         mg_coords(L, n, mx, my, k);
-        T acc = (T)0;
-        for (int m = 0; m < nz; ++m) acc += Qz[m * nz + k] * b[(mx * ny + my) * nz + m];
-        a[n] = acc;
+        a[n] = mg_dot(Qz + k, nz, b + (mx * ny + my) * nz, 1, nz);
     }
     __syncthreads();
     for (int n = tid; n < L.n; n += nt) {
         int mx, j, k;
         mg_coords(L, n, mx, j, k);
-        T acc = (T)0;
-        for (int m = 0; m < ny; ++m) acc += Qy[m * ny + j] * a[(mx * ny + m) * nz + k];
-        b[n] = acc;
+        b[n] = mg_dot(Qy + j, ny, a + mx * ny * nz + k, nz, ny);
     }
     __syncthreads();
     for (int n = tid; n < L.n; n += nt) {
         int i, j, k;
         mg_coords(L, n, i, j, k);
-        T acc = (T)0;
-        for (int m = 0; m < nx; ++m) acc += Qx[m * nx + i] * b[(m * ny + j) * nz + k];
-        L.u[n] = acc;
+        L.u[n] = mg_dot(Qx + i, nx, b + j * nz + k, ny * nz, nx);
     }
 }
 
-template <typename T>
-__global__ void __launch_bounds__(kMGCoarseThreads) k_mg_coarse(MGLevelT<T> L)
+// values of the exact solve's tables; they are copied to LDS where they are this few
+constexpr int kMGTableLds = 4096;
+template <typename T> __host__ __device__ inline int mg_table(const MGLevelT<T> &B)
 {
-    extern __shared__ double coarse_lds[];
-    T *a = reinterpret_cast<T *>(coarse_lds);
-    mg_coarse_solve(L, a, a + L.n);
+    return B.nx * B.nx + B.ny * B.ny + B.nz * B.nz + B.nx + B.ny + B.nz;
 }
 
-// The two coarsest levels in one workgroup: the level F above the coarsest (stored by
-// colour) from its first sweep to its last, with the restriction to the coarsest level
-// C, C's exact solve and the prolongation between.  These levels hold a few thousand
-// cells, where a launch per half sweep costs more than the sweep.  Here F's u (and its
-// f, where both fit in 64 KiB of LDS with C's two work arrays) stay in LDS from the
-// first step to the last, the steps a barrier apart, and only F's final u goes back to
-// global memory for the prolongation to the finer level.  Every cell is updated by the
-// same device function as in the per-step kernels (the restriction and prolongation by
-// their general forms, which give the same values as the z-only ones), so the result
-// is the same bits.
-constexpr size_t kMGTailLds = 65536;
+// The tail of the hierarchy in one workgroup: its first level (see kMGTailCells) and all
+// below it, from that level's first sweep to its last, the exact solve included.
+// These levels hold a few thousand cells, where a launch per half sweep costs more than
+// the sweep.  Every level's u and f stay in LDS, the steps a barrier apart; only the first
+// level's f comes from global memory and its u goes back.
 template <typename T>
-__host__ __device__ inline bool mg_tail_f_in_lds(int fn, int cn)
+struct MGTail {
+    MGLevelT<T> L[kMGTailLevels];
+    int nlev;
+};
+
+// half sweep of colour c over a level in LDS
+template <typename T>
+__device__ __forceinline__ void mg_tail_sweep(const MGLevelT<T> &L, int c)
 {
-    return (2 * (size_t)fn + 2 * (size_t)cn) * sizeof(T) <= kMGTailLds;
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const T *u = L.u;
+    auto cell = [&](int n, int i, int j, int k) {
+        const T s = mg_nbsum(L, n, i, j, k, [&](int q, int, int, int) { return u[q]; });
+        L.u[n] = (L.f[n] + s) / mg_diag(L, i, j, k);
+    };
+    if ((L.nz & 1) == 0) {
+        const int half = L.nz >> 1;
+        for (int m = tid; m < (L.n >> 1); m += nt) {
+            const int row = (int)fdiv((unsigned)m, L.dzh);
+            const int i = (int)fdiv((unsigned)row, L.dy), j = row - i * L.ny;
+            const int k = 2 * (m - row * half) + ((i + j + c) & 1);
+            cell(row * L.nz + k, i, j, k);
+        }
+    } else {
+        // periodic z joins two cells of one colour: their planes in turn (k_mg_smooth_cell)
+        const bool wrap_same = L.zper && L.nz > 1;
+        for (int pass = 0; pass < (wrap_same ? 2 : 1); ++pass) {
+            if (pass) __syncthreads();
+            for (int n = tid; n < L.n; n += nt) {
+                int i, j, k;
+                mg_coords(L, n, i, j, k);
+                if (((i + j + k) & 1) != c) continue;
+                if (wrap_same && (k == L.nz - 1) != (pass == 1)) continue;
+                cell(n, i, j, k);
+            }
+        }
+    }
+    __syncthreads();
 }
 
-template <typename T, bool F_LDS>
-__global__ void __launch_bounds__(kMGCoarseThreads) k_mg_tail(MGLevelT<T> F, MGLevelT<T> C)
+template <typename T>
+__global__ void __launch_bounds__(kMGCoarseThreads) k_mg_tail(MGTail<T> t)
 {
     extern __shared__ double coarse_lds[];
-    const int tid = threadIdx.x, nt = blockDim.x, hn = F.n >> 1;
-    T *su = reinterpret_cast<T *>(coarse_lds);
-    T *sf = su + F.n;
-    T *ca = F_LDS ? sf + F.n : sf, *cb = ca + C.n;
-    MGLevelT<T> FL = F, CL = C;
-    FL.u = su;
-    if (F_LDS) {
-        FL.f = sf;
-        for (int n = tid; n < F.n; n += nt) sf[n] = F.f[n];
+    const int tid = threadIdx.x, nt = blockDim.x, nl = t.nlev;
+    const int table = mg_table(t.L[nl - 1]);
+    T *tab = reinterpret_cast<T *>(coarse_lds);
+    T *mem = tab + (table <= kMGTableLds ? (table + 1) / 2 * 2 : 0);
+    for (int n = tid; n < t.L[0].n; n += nt) mem[t.L[0].n + n] = t.L[0].f[n];
+    if (table <= kMGTableLds)
+        for (int n = tid; n < table; n += nt) tab[n] = t.L[nl - 1].fd[n];
+    __syncthreads();
+    T *at = mem;
+    for (int l = 0; l < nl - 1; ++l) {
+        MGLevelT<T> F = t.L[l], C = t.L[l + 1];
+        F.u = at;
+        F.f = at + F.n;
+        at += 2 * F.n;
+        C.f = at + C.n;
+        // first red sweep from u = 0
+        for (int n = tid; n < F.n; n += nt) {
+            int i, j, k;
+            mg_coords(F, n, i, j, k);
+            F.u[n] = ((i + j + k) & 1) ? (T)0 : F.f[n] / mg_diag(F, i, j, k);
+        }
+        __syncthreads();
+        mg_tail_sweep(F, 1);
+        mg_tail_sweep(F, 0);
+        mg_tail_sweep(F, 1);
+        for (int m = tid; m < C.n; m += nt) mg_restrict_at(F, C, m);
         __syncthreads();
     }
-    // C's right-hand side is built in the first work array and its result left there
-    CL.f = ca;
-    CL.u = ca;
-    for (int m = tid; m < hn; m += nt) mg_smooth_first_at(FL, m);
-    __syncthreads();
-    for (int m = tid; m < hn; m += nt) mg_smooth_at(FL, m, 0);
-    __syncthreads();
-    for (int m = tid; m < hn; m += nt) mg_smooth_at(FL, m, 1);
-    __syncthreads();
-    for (int m = tid; m < C.n; m += nt) mg_restrict_at(FL, CL, m);
-    __syncthreads();
-    mg_coarse_solve(CL, ca, cb);
-    __syncthreads();
-    for (int m = tid; m < hn; m += nt) mg_prolong_smooth_at(FL, CL, m);
-    __syncthreads();
-    for (int m = tid; m < hn; m += nt) mg_smooth_at(FL, m, 1);
-    __syncthreads();
-    for (int m = tid; m < hn; m += nt) mg_smooth_at(FL, m, 0);
-    __syncthreads();
-    for (int m = tid; m < hn; m += nt) mg_smooth_at(FL, m, 1);
-    __syncthreads();
-    for (int n = tid; n < F.n; n += nt) F.u[n] = su[n];
+    {
+        MGLevelT<T> B = t.L[nl - 1];
+        B.f = at + B.n;
+        B.u = at;
+        if (table <= kMGTableLds) mg_coarse_solve(B, (const T *)tab, at, at + B.n);
+        else mg_coarse_solve(B, B.fd, at, at + B.n);
+        __syncthreads();
+    }
+    for (int l = nl - 2; l >= 0; --l) {
+        MGLevelT<T> F = t.L[l], C = t.L[l + 1];
+        C.u = at;
+        at -= 2 * F.n;
+        F.u = at;
+        F.f = at + F.n;
+        for (int n = tid; n < F.n; n += nt) mg_prolong_at(F, C, n);
+        __syncthreads();
+        mg_tail_sweep(F, 0);
+        mg_tail_sweep(F, 1);
+        mg_tail_sweep(F, 0);
+        mg_tail_sweep(F, 1);
+    }
+    for (int n = tid; n < t.L[0].n; n += nt) t.L[0].u[n] = mem[n];
 }
 
 // ---- preconditioned BiCGSTAB pieces (linear cell order, canonical block sums) ----
@@ -825,62 +569,174 @@ __global__ void __launch_bounds__(kThreads) k_pb_end(Geo g, const double *part, 
 }
 
 // ---- launchers ----
+template <typename T, int P> static size_t sweep_lds(const MGSweepT<T> &a);
+
+template <typename T, int P, bool ZPER>
+static void launch_sweep(hipStream_t s, const MGSweepT<T> &a, bool down)
+{
+    const int threads = 2 * mg_half_block(a.rows, a.tpr);
+    const size_t lds = sweep_lds<T, P>(a);
+    const dim3 grid((a.nblk + 7) / 8 * 8);
+    if (!down) {
+        if (a.fz == 2)
+            hipLaunchKernelGGL((k_mg_up<T, P, ZPER, true>), grid, dim3(threads), lds, s, a);
+        else
+            hipLaunchKernelGGL((k_mg_up<T, P, ZPER, false>), grid, dim3(threads), lds, s, a);
+    } else if (a.fx == 1 && a.fy == 1 && a.fz == 2) {
+        hipLaunchKernelGGL((k_mg_down<T, P, ZPER, 0>), grid, dim3(threads), lds, s, a);
+    } else {
+        hipLaunchKernelGGL((k_mg_down<T, P, ZPER, 1>), grid, dim3(threads), lds, s, a);
+    }
+}
+
+// The tiling of a level for the one-pass kernels, from an estimate of a block's step: a CU
+// with W waves resident takes lat + add W us for a plane, or W issue us where the
+// instructions bound it (fitted to both kernels over 15 level shapes from 96x48x6 to
+// 1024x512x128, every P, ty and cxl: the choice is within 0.3% of the best measured one in
+// the mean).  More rows and planes a block mean fewer formed twice; more blocks fill the CUs.
+struct SweepCost {
+    double lat, add, issue;
+    int waves; // of this kernel a CU holds (registers)
+};
+template <typename T, int P> static SweepCost sweep_cost()
+{
+    if (std::is_same<T, float>::value)
+        return P == 1 ? SweepCost{0.45, 0.012, 0.054, 16}
+                      : (P == 2 ? SweepCost{0.63, 0.008, 0.070, 8}
+                                : SweepCost{0.86, 0.020, 0.133, 8});
+    return P == 1 ? SweepCost{0.45, 0.035, 0.060, 8} : SweepCost{0.74, 0.039, 0.134, 8};
+}
+
+template <typename T, int P>
+static size_t sweep_lds(const MGSweepT<T> &a)
+{
+    return 8 * (size_t)a.rows * mg_lds_row<P>(a.pairs) * sizeof(T) +
+           (a.fy == 2 ? 4 * (size_t)a.rows * a.pairs * sizeof(T) : 0);
+}
+
+template <typename T, int P>
+static void sweep_tiles(MGSweepT<T> &a, int ty, int tz, int cxl)
+{
+    a.ty = ty;
+    a.rows = ty + 2 * kMGHalo;
+    a.tz = tz;
+    a.nkt = cdiv(a.half, tz);
+    a.pairs = a.nkt == 1 ? a.half : tz + 2 * mg_zhalo<P>();
+    a.tpr = a.pairs / P;
+    a.cxl = cxl;
+    a.njt = cdiv(a.ny, ty);
+    a.nblk = a.njt * a.nkt * cdiv(a.nx, cxl);
+}
+
+template <typename T, int P>
+static void sweep_try(const MGSweepT<T> &base, double &best, MGLevelT<T> &F)
+{
+    if (base.half % P) return;
+    const SweepCost c = sweep_cost<T, P>();
+    MGSweepT<T> a = base;
+    for (int tz : {base.half, 64, 32}) {
+        if (tz < base.half && base.half <= kMGLongRow) break;
+        if (tz > base.half) continue;
+        for (int ty : {2, 4, 8, 16, 24, 32, 40, 56, 64, 120}) {
+            if (ty > 2 && ty - 8 >= base.ny) break;
+            sweep_tiles<T, P>(a, ty, tz, 2);
+            const int waves = 2 * mg_half_block(a.rows, a.tpr) / 64;
+            const size_t lds = sweep_lds<T, P>(a);
+            if (waves * 64 > kMGSweepThreads || lds > kMGSweepLds) break;
+            const int fit = std::max(1, std::min(c.waves / waves, (int)(kMGSweepLds / lds)));
+            auto step = [&](int blocks) {
+                const double w = (double)blocks * waves;
+                return std::max(c.lat + c.add * w, c.issue * w);
+            };
+            for (int cxl : {2, 4, 6, 8, 12, 16, 20, 24, 28, 32, 48, 64, 96, 128, 256, 512}) {
+                if (cxl > 2 && cxl >= 2 * base.nx) break;
+                sweep_tiles<T, P>(a, ty, tz, cxl);
+                const int per_cu = cdiv(a.nblk, 256), full = per_cu / fit, rest = per_cu % fit;
+                const double t =
+                    (cxl + 2 * kMGHalo) * (full * step(fit) + (rest ? step(rest) : 0.0));
+                if (t < best) {
+                    best = t;
+                    F.sp = P, F.sty = ty, F.stz = tz, F.scx = cxl;
+                }
+            }
+        }
+    }
+}
+
+template <typename T>
+static MGSweepT<T> sweep_args(const MGLevelT<T> &F, const MGLevelT<T> &C)
+{
+    MGSweepT<T> a = {};
+    a.nx = F.nx, a.ny = F.ny, a.nz = F.nz, a.half = F.nz >> 1;
+    a.fx = C.fx, a.fy = C.fy, a.fz = C.fz, a.cny = C.ny, a.cnz = C.nz;
+    a.cx = F.cx, a.cy = F.cy, a.cz = F.cz;
+    a.f = F.f, a.e = C.u, a.ub = F.ub, a.fc = C.f, a.u = F.u;
+    return a;
+}
+
+template <typename T>
+void mg_plan(MGLevelT<T> *L, int nlev)
+{
+    for (int l = 0; l + 1 < nlev; ++l) {
+        L[l].sp = 0;
+        if (L[l].nz & 1) continue; // odd nz: a launch per half sweep
+        const MGSweepT<T> a = sweep_args(L[l], L[l + 1]);
+        double best = 1e30;
+        sweep_try<T, 1>(a, best, L[l]);
+        sweep_try<T, 2>(a, best, L[l]);
+        if (std::is_same<T, float>::value) sweep_try<T, 4>(a, best, L[l]);
+    }
+}
+
+template <typename T>
+static void launch_half_cycle(hipStream_t s, const MGLevelT<T> &F, const MGSweepT<T> &a, int P,
+                              bool down)
+{
+    auto go = [&](auto zper) {
+        constexpr bool Z = decltype(zper)::value;
+        if constexpr (std::is_same<T, float>::value) {
+            if (P == 4) return launch_sweep<T, 4, Z>(s, a, down);
+        }
+        if (P == 2) launch_sweep<T, 2, Z>(s, a, down);
+        else launch_sweep<T, 1, Z>(s, a, down);
+    };
+    if (F.zper) go(std::true_type());
+    else go(std::false_type());
+}
+
+// LDS of the tail from level l on; 0 where level l does not start it
+template <typename T>
+static size_t tail_lds(const MGLevelT<T> *L, int nlev, int l)
+{
+    if (l < nlev - 1 && (L[l].n > ((L[l].nz & 1) ? kMGTailCellsOdd : kMGTailCells) ||
+                         nlev - l > kMGTailLevels))
+        return 0;
+    const int table = mg_table(L[nlev - 1]);
+    size_t n = table <= kMGTableLds ? (table + 1) / 2 * 2 : 0;
+    for (int q = l; q < nlev; ++q) n += 2 * (size_t)L[q].n;
+    return n * sizeof(T);
+}
+
 template <typename T>
 void launch_mg_vcycle(hipStream_t s, const MGLevelT<T> *L, int nlev, int l)
 {
     const MGLevelT<T> &F = L[l];
-    if (l == nlev - 1) {
-        hipLaunchKernelGGL(k_mg_coarse<T>, dim3(1), dim3(kMGCoarseThreads),
-                           2 * (size_t)F.n * sizeof(T), s, F);
+    if (const size_t lds = tail_lds(L, nlev, l)) {
+        MGTail<T> t;
+        t.nlev = nlev - l;
+        for (int q = l; q < nlev; ++q) t.L[q - l] = L[q];
+        hipLaunchKernelGGL(k_mg_tail<T>, dim3(1), dim3(kMGCoarseThreads), lds, s, t);
         return;
     }
     const MGLevelT<T> &C = L[l + 1];
-    const size_t tail_lds =
-        ((mg_tail_f_in_lds<T>(F.n, C.n) ? 2 : 1) * (size_t)F.n + 2 * (size_t)C.n) * sizeof(T);
-    if (l > 0 && l == nlev - 2 && (F.nz & 1) == 0 && F.n <= kMGTailCells &&
-        tail_lds <= kMGTailLds) {
-        if (mg_tail_f_in_lds<T>(F.n, C.n))
-            hipLaunchKernelGGL((k_mg_tail<T, true>), dim3(1), dim3(kMGCoarseThreads), tail_lds, s,
-                               F, C);
-        else
-            hipLaunchKernelGGL((k_mg_tail<T, false>), dim3(1), dim3(kMGCoarseThreads), tail_lds, s,
-                               F, C);
-        return;
-    }
-    if ((F.nz & 1) == 0) {
-        const int nb = cdiv(F.n >> 1, 256);
-        // a plain half sweep: in FP64 two cells of a colour per thread where rows hold
-        // whole pairs (measured 4% faster per V-cycle at 512x256x64); in FP32 one cell per
-        // thread (pairs measured 3% slower there, four cells level with one)
-        auto smooth = [&](int colour) {
-            if constexpr (std::is_same<T, double>::value) {
-                if ((F.nz & 3) == 0) {
-                    hipLaunchKernelGGL(k_mg_smooth2<T>, dim3(cdiv(F.n >> 2, 256)), dim3(256), 0,
-                                       s, F, colour);
-                    return;
-                }
-            }
-            hipLaunchKernelGGL(k_mg_smooth<T>, dim3(nb), dim3(256), 0, s, F, colour);
-        };
-        hipLaunchKernelGGL(k_mg_smooth_first<T>, dim3(nb), dim3(256), 0, s, F);
-        smooth(0);
-        smooth(1);
-        const bool zonly = C.fx == 1 && C.fy == 1 && C.fz == 2;
-        if (zonly)
-            hipLaunchKernelGGL(k_mg_restrict_z<T>, dim3(nb), dim3(256), 0, s, F, C);
-        else
-            hipLaunchKernelGGL(k_mg_restrict<T>, dim3(cdiv(C.n, 256)), dim3(256), 0, s, F, C);
+    if (F.sp) {
+        MGSweepT<T> a = sweep_args(F, C);
+        if (F.sp == 4) sweep_tiles<T, 4>(a, F.sty, F.stz, F.scx);
+        else if (F.sp == 2) sweep_tiles<T, 2>(a, F.sty, F.stz, F.scx);
+        else sweep_tiles<T, 1>(a, F.sty, F.stz, F.scx);
+        launch_half_cycle(s, F, a, F.sp, true);
         launch_mg_vcycle(s, L, nlev, l + 1);
-        if (zonly)
-            hipLaunchKernelGGL(k_mg_prolong_smooth_z<T>, dim3(nb), dim3(256), 0, s, F, C);
-        else
-            hipLaunchKernelGGL(k_mg_prolong_smooth<T>, dim3(nb), dim3(256), 0, s, F, C);
-        smooth(1);
-        smooth(0);
-        if (F.uout)
-            hipLaunchKernelGGL(k_mg_smooth_out<T>, dim3(nb), dim3(256), 0, s, F);
-        else
-            smooth(1);
+        launch_half_cycle(s, F, a, F.sp, false);
         return;
     }
     const int nb = cdiv(F.n, 256);
@@ -973,6 +829,7 @@ void launch_pb_end(const Geo &g, hipStream_t s, const double *part, PBState *st)
 }
 
 #define CFDMX_MG_INSTANCES(T)                                                                 \
+    template void mg_plan<T>(MGLevelT<T> *, int);                                             \
     template void launch_mg_vcycle<T>(hipStream_t, const MGLevelT<T> *, int, int);            \
     template void launch_pb_spmv<T>(const Geo &, hipStream_t, const MGLevelT<T> &, int,       \
                                     const T *, T *, const T *, double *, const PBState *);    \
