@@ -97,6 +97,12 @@ struct cfdmx_ctx {
     // factor (Cs delta)^2
     double *viseff = nullptr, *smag_coef = nullptr;
     double *bpart[3] = {}; // per-phase BiCGSTAB partials (A, B, C)
+    // resident BiCGSTAB (cfdmx_bicg_grid.hip): where the grid takes it, its partial sums'
+    // slots and its failure flag
+    int grid_solve = 0, grid_uni = 0;
+    unsigned long long *grid_slots = nullptr;
+    KState *grid_keep = nullptr;
+    int *grid_failed = nullptr, *grid_failed_h = nullptr;
     double *scal = nullptr; // [0] cfl, [1] cd, [2] cl, [3..5] max(T0 - T3) of u, v, w
     double *inflow = nullptr;
     KState *kst = nullptr;
@@ -148,6 +154,8 @@ static __device__ __align__(256) double scratch[2 * kScratchBlocks];
 constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
 static double *g_scratch[kMaxDevices] = {};
+// one resident BiCGSTAB kernel at a time on a device (solve_bicgstab_core)
+static std::mutex g_grid_mu[kMaxDevices];
 
 #define FAIL(code, ...)                                                                        \
     do {                                                                                       \
@@ -682,6 +690,21 @@ static int setup_device(cfdmx_ctx *ctx)
         HIPCHK(hipMemset(ctx->viseff, 0, N * sizeof(double)));
     }
     for (int q = 0; q < 3; ++q) ALLOC(ctx->bpart[q], 2 * (size_t)g.nmarch + 64);
+    // one set of coefficients for every row, whole tiles and whole blocks of planes
+    ctx->grid_uni = c.nx % kChunk == 0 && (g.cyz % kTile == 0 || g.cyz == 256 || g.cyz == 512);
+    for (int a = 0; a < 3; ++a)
+        for (int q = 0; q < 2; ++q)
+            for (int i = 0; i < nc[a]; ++i)
+                if (buf[poff[a][q] + i] != buf[poff[a][q]]) ctx->grid_uni = 0;
+    ctx->grid_solve =
+        c.precision == CFDMX_PRECISION_FP64 && bicg_grid_fits(g, c.precond, ctx->grid_uni) ? 1 : 0;
+    if (ctx->grid_solve) {
+        ALLOC(ctx->grid_slots, (size_t)bicg_grid_slots(g));
+        ALLOC(ctx->grid_keep, 1);
+        ALLOC(ctx->grid_failed, 1);
+        HIPCHK(hipMemset(ctx->grid_failed, 0, sizeof(int)));
+        HIPCHK(hipHostMalloc((void **)&ctx->grid_failed_h, sizeof(int), hipHostMallocDefault));
+    }
     ALLOC(ctx->flux_part, 3 * ((size_t)g.cyz / kPerBlock + 2));
     ALLOC(ctx->scal, 16);
     ALLOC(ctx->inflow, (size_t)g.ny);
@@ -878,6 +901,7 @@ int cfdmx_destroy(cfdmx_ctx *ctx)
     for (void *p : ctx->allocs) (void)hipFree(p);
     prof_harvest(ctx);
     for (hipEvent_t e : ctx->prof_pool) (void)hipEventDestroy(e);
+    if (ctx->grid_failed_h) (void)hipHostFree(ctx->grid_failed_h);
     if (ctx->kst_h) (void)hipHostFree(ctx->kst_h);
     if (ctx->pbs_h) (void)hipHostFree(ctx->pbs_h);
     for (void *q : ctx->adj.mem) (void)hipFree(q);
@@ -1246,7 +1270,46 @@ static int solve_bicgstab_core(cfdmx_ctx *ctx, const SolveTarget &T, int *iters,
     PROF(CFDMX_K_BICG_CHECK, launch_bicg_fin0(g, s, ctx->part, T.kst));
     LAUNCHCHK();
     int batch = 4, m = 0;
-    for (;;) {
+    // one resident kernel where the grid takes it, for as many iterations as one launch may
+    // last (11 to 31 us each); a solve that ends earlier ends the kernel
+    while (ctx->grid_solve) {
+        constexpr int kGridBatch = 1024;
+        hipError_t e = hipSuccess;
+        {
+            // two resident kernels of a device might each hold CUs that the other waits for
+            std::lock_guard<std::mutex> one(
+                g_grid_mu[ctx->device >= 0 && ctx->device < kMaxDevices ? ctx->device : 0]);
+            PROF(CFDMX_K_BICG_A,
+                 e = launch_bicg_grid(g, s, pre, ctx->grid_uni, ctx->B, T.x, ctx->bpart[2],
+                                      ctx->grid_slots, T.kst, ctx->grid_keep, ctx->grid_failed, m,
+                                      kGridBatch));
+            if (e == hipSuccess) {
+                HIPCHK(hipMemcpyAsync(T.kst_h, T.kst, sizeof(KState), hipMemcpyDeviceToHost, s));
+                HIPCHK(hipMemcpyAsync(ctx->grid_failed_h, ctx->grid_failed, sizeof(int),
+                                      hipMemcpyDeviceToHost, s));
+            }
+            HIPCHK(hipStreamSynchronize(s));
+        }
+        prof_harvest(ctx);
+        if (e != hipSuccess || *ctx->grid_failed_h) {
+            // its blocks were not all resident (another process's resident kernel, say): this
+            // solve again from its start, this context's solves by launched phases from here
+            (void)hipGetLastError();
+            ctx->grid_solve = 0;
+            *ctx->grid_failed_h = 0;
+            launch_set_int(s, ctx->grid_failed, 0);
+            launch_copy(s, g.N, *T.px1, T.x);
+            HIPCHK(hipMemcpyAsync(T.kst, ctx->grid_keep, sizeof(KState), hipMemcpyDeviceToDevice,
+                                  s));
+            launch_bicg_init(g, s, pre, T.b, T.x, ctx->B.r0, ctx->B.r, *T.px1, ctx->part, T.kst);
+            LAUNCHCHK();
+            m = 0;
+            break;
+        }
+        m += kGridBatch;
+        if (T.kst_h->done) break;
+    }
+    while (!ctx->grid_solve) {
         for (int q = 0; q < batch; ++q, ++m) {
             PROF(CFDMX_K_BICG_A, launch_bicg_A(g, s, pre, ctx->B, ctx->bpart, T.kst, m));
             PROF(CFDMX_K_BICG_B, launch_bicg_B(g, s, pre, ctx->B, ctx->bpart, T.kst, m));

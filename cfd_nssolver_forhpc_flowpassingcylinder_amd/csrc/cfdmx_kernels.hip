@@ -4,7 +4,7 @@
 // same association; the library is compiled with -ffp-contract=off and divisions
 // by grid metrics use the exactly rounded divr), so results equal the CPU
 // restatement bit for bit; sums use the canonical order of cfdmx_device.hpp.
-#include "cfdmx_internal.hpp"
+#include "cfdmx_bicg.hpp"
 
 namespace cfdmx {
 
@@ -1092,65 +1092,12 @@ struct MarchIO {
     double *part;
 };
 
-// planes of march block `chunk`: first plane and direction
-__device__ __forceinline__ void march_span(const Geo &g, int chunk, int &first, int &dir, int &len)
-{
-    const int i0 = chunk * kChunk, i1 = min(i0 + kChunk, g.nxc);
-    len = i1 - i0;
-    dir = (chunk & 1) ? 1 : -1;
-    first = dir > 0 ? i0 : i1 - 1;
-}
-
 // LDS of a march block: x coefficients of the chunk's planes, y coefficients of the
 // tile's rows, z coefficients (double), then two plane slots (T)
 __host__ __device__ inline int march_rows(int nzc) { return kTile / nzc + 2; }
 
-template <int PRE>
-__device__ __forceinline__ void march_row(const Geo &g, int i, int j, int k, double xm, double xp,
-                                          double ym, double yp, double zm, double zp,
-                                          double v[7])
-{
-    if (PRE == 0) {
-        double ijk = xm + ym + zm + xp + yp + zp;
-        if (i == 0) ijk -= xm;
-        if (i == g.nxc - 1) ijk -= xp;
-        if (j == 0) ijk -= ym;
-        if (j == g.nyc - 1) ijk -= yp;
-        if (!g.zper) {
-            if (k == 0) ijk -= zm;
-            if (k == g.nzc - 1) ijk -= zp;
-        }
-        v[0] = -xm;
-        v[1] = -yp;
-        v[2] = -zm;
-        v[3] = ijk;
-        v[4] = -zp;
-        v[5] = -ym;
-        v[6] = -xp;
-    } else {
-        double aa = 0.0, bb = 0.0, cc = 0.0;
-        if (i == 0) aa = -xm;
-        if (i == g.nxc - 1) aa = -xp;
-        if (j == 0) bb = -ym;
-        if (j == g.nyc - 1) bb = -yp;
-        if (!g.zper) {
-            if (k == 0) cc = -zm;
-            if (k == g.nzc - 1) cc = -zp;
-        }
-        const double ijk = xm + ym + zm + xp + yp + zp + aa + bb + cc;
-        const double jp = 1.0 / ijk;
-        v[0] = -xm * jp;
-        v[1] = -ym * jp;
-        v[2] = -zm * jp;
-        v[3] = ijk * jp;
-        v[4] = -zp * jp;
-        v[5] = -yp * jp;
-        v[6] = -xp * jp;
-    }
-}
-
-// Start of iteration m in phase A: the end of iteration m-1 (bicgstabRe2.hpp:129-174)
-// from phase C's partials (r,r), (r,r0).  Returns false when the solve has ended.
+// Start of iteration m in phase A, from phase C's partials.  Returns false when the solve
+// has ended.
 __device__ __forceinline__ bool bicg_iteration_start(const Geo &g, KState *st, int m,
                                                      const double *partC, bool writer,
                                                      int &mode, double &beta)
@@ -1162,40 +1109,27 @@ __device__ __forceinline__ bool bicg_iteration_start(const Geo &g, KState *st, i
     }
     double t[2];
     fold_partials<2>(partC, g.nmarch, g.nmarch, t);
-    const double res = sqrt(t[0]) / st->norm0; // L2Norm(r1) / norm0
-    const int it = m - 1;                      // pIter of the iteration that just ended
-    if (res < st->tol || it >= st->maxit) {
+    BicgNext o;
+    if (!bicg_next(t, st->norm0, st->tol, st->restart_factor, st->maxit, st->timestep, m,
+                   st->alpha, st->omega, st->rho[(m - 1) & 1], o)) {
         if (writer) {
-            st->res = res;
-            st->iter = it;
-            st->done = res < st->tol ? 1 : 2;
+            st->res = o.res;
+            st->iter = m - 1;
+            st->done = o.res < st->tol ? 1 : 2;
         }
         return false;
     }
-    const double rho_l = st->rho[(m - 1) & 1];
-    const double rho = t[1];
-    beta = (st->alpha / st->omega) * (rho / rho_l);
-    mode = (st->timestep < 10 || fabs(rho_l) > st->tol * st->restart_factor) ? 0 : 1;
+    mode = o.mode;
+    beta = o.beta;
     if (writer) {
-        st->rho[m & 1] = rho;
-        st->res = res;
+        st->rho[m & 1] = t[1];
+        st->res = o.res;
         st->iter = m;
         st->beta = beta;
         st->mode = mode;
         if (mode == 1) st->restarts += 1;
     }
     return true;
-}
-
-// v when ok is 1, +0 when ok is 0, by masking the bits (a select here becomes a branch
-// around the LDS store, which costs the plane loop its overlap of loads and stores)
-__device__ __forceinline__ double keep_if(double v, int ok)
-{
-    return __longlong_as_double(__double_as_longlong(v) & -(long long)ok);
-}
-__device__ __forceinline__ float keep_if(float v, int ok)
-{
-    return __int_as_float(__float_as_int(v) & -ok);
 }
 
 // A march block keeps the new vector (p for A, s for B) of its own cells on the planes
@@ -1389,7 +1323,14 @@ k_march(Geo g, MarchIO<T> io, KState *st, int m, const double *part_in)
             if (!FULL && tq >= qn) break;
             const int jj = jc[c], k = kc[c], j = jlo + jj;
             double v[7];
-            march_row<PRE>(g, i, j, k, xm, xp, cy[jj], cy[RY + jj], cz[k], cz[g.nzc + k], v);
+            const double ym = cy[jj], yp = cy[RY + jj], zm = cz[k], zp = cz[g.nzc + k];
+            const RowEnds end = {i == 0 ? xm : 0.0,
+                                 i == g.nxc - 1 ? xp : 0.0,
+                                 j == 0 ? ym : 0.0,
+                                 j == g.nyc - 1 ? yp : 0.0,
+                                 !g.zper && k == 0 ? zm : 0.0,
+                                 !g.zper && k == g.nzc - 1 ? zp : 0.0};
+            march_row<PRE>(end, xm, xp, ym, yp, zm, zp, v);
             // All neighbour reads are unconditional (the halo rows and the zeroed
             // planes outside the grid are in place), and a missing neighbour adds +0.0
             // in place of its term.  The running sum starts at +0.0 and so is never

@@ -313,7 +313,7 @@ CFDMX_API int cfdmx_adjoint_drag(cfdmx_ctx *ctx, int nsteps, int checkpoint_ever
 #define CFDMX_K_BC 1
 #define CFDMX_K_RHS 2
 #define CFDMX_K_BICG_INIT 3
-#define CFDMX_K_BICG_A 4
+#define CFDMX_K_BICG_A 4 /* the whole solve where one resident kernel runs it (B and C then stay 0) */
 #define CFDMX_K_BICG_B 5
 #define CFDMX_K_BICG_C 6
 #define CFDMX_K_BICG_CHECK 7 /* initial fold and end-of-batch convergence check */
