@@ -131,6 +131,8 @@ struct cfdmx_ctx {
     // red-black SOR working set of a context configured for it (even nzc): p of both
     // colours, then the right-hand side of both colours, in one allocation
     double *sorw = nullptr;
+    SorState *sorst = nullptr;
+    SorPlan sorp = {}; // passes of two sweeps, in contexts configured for red-black SOR
     int *count = nullptr;
     // pinned host mirrors
     KState *kst_h = nullptr;
@@ -687,7 +689,18 @@ static int setup_device(cfdmx_ctx *ctx)
     ALLOC(ctx->B.q, N);
     ALLOC(ctx->B.p, N);
     ALLOC(ctx->B.ap, N);
-    if (ctx->cfg.solver == CFDMX_SOLVER_RBSOR && g.nzc % 2 == 0) ALLOC(ctx->sorw, 2 * N);
+    if (ctx->cfg.solver == CFDMX_SOLVER_RBSOR) {
+        int dev = 0, cus = 0;
+        HIPCHK(hipGetDevice(&dev));
+        HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        ctx->sorp = sor_plan(g, ctx->sorc, cus);
+        if (ctx->sorp.blocks) {
+            ALLOC(ctx->sorw, G + G % 2 + N + 4 * (size_t)ctx->sorp.blocks);
+            ALLOC(ctx->sorst, 2);
+        } else if (g.nzc % 2 == 0) {
+            ALLOC(ctx->sorw, 2 * N);
+        }
+    }
     ALLOC(ctx->part, 4 * (size_t)(g.nblocks > g.nmarch ? g.nblocks : g.nmarch) + 64);
     ALLOC(ctx->cfl_part, (size_t)g.cd_nb + 8);
     ALLOC(ctx->diff_part, 3 * (size_t)g.nblocks + 8);
@@ -1648,6 +1661,44 @@ int cfdmx_solve_bicgstab(cfdmx_ctx *ctx, int *iters, double *residual)
     return solve_bicgstab_impl(ctx, iters, residual);
 }
 
+// passes of two sweeps, p and a copy of it in turn; the state says after which sweep to end
+static int solve_rbsor_passes(cfdmx_ctx *ctx)
+{
+    hipStream_t s = ctx->stream;
+    const Geo &g = ctx->g;
+    const SorPlan &pl = ctx->sorp;
+    double *buf[2] = {ctx->p, ctx->sorw};
+    double *rhs = ctx->sorw + g.G + g.G % 2;
+    double *part[2] = {rhs + g.N, rhs + g.N + 2 * (size_t)pl.blocks};
+    const auto pass = [&](int from, const SorTurn &turn) {
+        PROF(CFDMX_K_SOR, launch_sor_pass(g, s, pl, ctx->cfg.sor_omega, ctx->sorc, rhs,
+                                          buf[from], buf[from ^ 1], turn));
+    };
+    PROF(CFDMX_K_RHS, launch_sor_rhs(g, s, ctx->t1[0], ctx->t1[1], ctx->t1[2], ctx->cfg.dt, rhs));
+    launch_copy(s, g.G, buf[0], buf[1]);
+    LAUNCHCHK();
+    for (int batch = 2;; batch = batch < 32 ? batch * 2 : 32) { // an even number of passes
+        for (int q = 0; q < batch; ++q) {
+            const int h = q & 1;
+            pass(h, {q ? ctx->sorst + (h ^ 1) : ctx->sst, q ? part[h ^ 1] : nullptr,
+                     ctx->sorst + h, part[h], 2});
+        }
+        launch_sor_pass_fin(s, pl, ctx->sorst + 1, part[1], ctx->sst);
+        LAUNCHCHK();
+        HIPCHK(hipMemcpyAsync(ctx->sst_h, ctx->sst, sizeof(SorState), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipStreamSynchronize(s));
+        prof_harvest(ctx);
+        if (ctx->sst_h->done) break;
+    }
+    // the last pass read p or the copy as it was the ((iters - 1) / 2)-th or not; if its first
+    // sweep was the last one, that sweep alone is run again from there
+    const int from = ((ctx->sst_h->iters - 1) / 2) & 1;
+    if (ctx->sst_h->iters & 1) pass(from, {nullptr, nullptr, nullptr, part[0], 1});
+    if (from == 0) launch_copy(s, g.G, buf[1], buf[0]);
+    LAUNCHCHK();
+    return CFDMX_OK;
+}
+
 static int solve_rbsor_impl(cfdmx_ctx *ctx, int *iters, double *err)
 {
     hipStream_t s = ctx->stream;
@@ -1657,6 +1708,12 @@ static int solve_rbsor_impl(cfdmx_ctx *ctx, int *iters, double *err)
     ss.itmax = ctx->cfg.maxit;
     *ctx->sst_h = ss;
     HIPCHK(hipMemcpyAsync(ctx->sst, ctx->sst_h, sizeof ss, hipMemcpyHostToDevice, s));
+    if (ctx->sorp.blocks) {
+        if (int rc = solve_rbsor_passes(ctx)) return rc;
+        if (iters) *iters = ctx->sst_h->iters - 1; // SorPipeLine.seq.hpp:123
+        if (err) *err = ctx->sst_h->residual;
+        return CFDMX_OK;
+    }
     // even nzc: colour-split storage, p's natural order written back at the end; the
     // working set is the context's own when it is configured for red-black SOR, else the
     // Krylov vector r0 (p of both colours) and b (the right-hand side).  Odd nzc: the

@@ -48,6 +48,16 @@ struct SorState {
     int pad;
 };
 
+// tiles of the pass that runs two red-black sweeps at once (cfdmx_sor.hip); blocks is 0 on
+// grids it does not take
+struct SorPlan {
+    int width, threads;  // pairs of a tile's row with their halo, threads of a block
+    int cown, ntz;       // pairs of k a block owns, pieces of a row
+    int yown, nty;       // rows a block owns, tiles of rows
+    int xlen, ntx;       // planes a block owns, spans of planes
+    int blocks;
+};
+
 // Krylov vectors of one BiCGSTAB solve.  q holds p - omega*Ap between phase C and the
 // next phase A.  p is written by phase A for phase C only on grids whose vectors fit the
 // caches; above that C forms it again from r and q (k_march_C).
@@ -185,6 +195,23 @@ void launch_extrapolate(const Geo &g, hipStream_t s, double *x, double *xp);
 void launch_fill(hipStream_t s, int n, double val, double *a);
 void launch_sor_rhs(const Geo &g, hipStream_t s, const double *us, const double *vs,
                     const double *ws, double dt, double *cf6);
+SorPlan sor_plan(const Geo &g, const SorCoef &sc, int cus);
+// two sweeps from src into dst (one: sweeps = 1, which looks at no state), unless the state
+// `in`, advanced by the pass that left its maxima in `was` (null: none), says done; the state
+// goes to `out`, this pass's maxima (2 * blocks) to `part`
+struct SorTurn {
+    const SorState *in;
+    const double *was;
+    SorState *out;
+    double *part;
+    int sweeps;
+};
+void launch_sor_pass(const Geo &g, hipStream_t s, const SorPlan &pl, double omega,
+                     const SorCoef &sc, const double *rhs, const double *src, double *dst,
+                     const SorTurn &turn);
+// the state `in` advanced by the maxima in `part`
+void launch_sor_pass_fin(hipStream_t s, const SorPlan &pl, const SorState *in,
+                         const double *part, SorState *out);
 void launch_sor_half(const Geo &g, hipStream_t s, int colour, double omega, const double *cf6,
                      double *p, double *part, SorState *st);
 void launch_sor_fin(const Geo &g, hipStream_t s, double *part, SorState *st);
