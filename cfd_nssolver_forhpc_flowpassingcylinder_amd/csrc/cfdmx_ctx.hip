@@ -68,7 +68,7 @@ struct cfdmx_ctx {
     };
     std::vector<VGraph> vgraphs;
     double *pb_part = nullptr;
-    double *mix = nullptr, *mix_h = nullptr;
+    double *mix_h = nullptr; // pinned: the three folded sums of the FP64 residual
     int mix_outer = 0;
     // Plot3D q output: staged float arrays on the device, pinned host copy filled on a
     // second stream, the file written when the next output or a flush comes
@@ -525,7 +525,6 @@ template <typename T> static int setup_multigrid(cfdmx_ctx *ctx)
     mg_plan(lev.data(), (int)lev.size());
     ALLOC(ctx->pbs, 1);
     ALLOC(ctx->pb_part, 2 * (size_t)g.nblocks + 64);
-    ALLOC(ctx->mix, 4);
     HIPCHK(hipHostMalloc((void **)&ctx->pbs_h, sizeof(PBState), hipHostMallocDefault));
     HIPCHK(hipHostMalloc((void **)&ctx->mix_h, 4 * sizeof(double), hipHostMallocDefault));
     return CFDMX_OK;
@@ -1558,9 +1557,8 @@ static int solve_pb_inner(cfdmx_ctx *ctx, double rr, double tol, int maxit, int 
         PROF(CFDMX_K_PB, launch_pb_spmv<T>(g, s, L[0], 2, sh, t, sv, ctx->part, ctx->pbs));
         PROF(CFDMX_K_PB, launch_pb_update_xr<T>(g, s, it == 0, ctx->part, ph, sh, sv, t, r0, e,
                                                 r, ctx->pb_part, ctx->pbs));
-        launch_pb_end(g, s, ctx->pb_part, ctx->pbs);
+        launch_pb_end(g, s, ctx->pb_part, ctx->pbs, ctx->pbs_h);
         LAUNCHCHK();
-        HIPCHK(hipMemcpyAsync(ctx->pbs_h, ctx->pbs, sizeof(PBState), hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
         prof_harvest(ctx);
     }
@@ -1581,10 +1579,8 @@ static int solve_refine(cfdmx_ctx *ctx, const double *b, double *x, int *iters, 
     // start (T(r), T(r)) in rr
     auto residual = [&](double &rr, double &rel) -> int {
         PROF(CFDMX_K_BICG_INIT, launch_mixed_resid<T>(g, s, 0, b, x, pv[0], pv[1], ctx->part));
-        launch_mixed_fold(g, s, ctx->part, ctx->mix);
+        launch_mixed_fold(g, s, ctx->part, ctx->mix_h);
         LAUNCHCHK();
-        HIPCHK(hipMemcpyAsync(ctx->mix_h, ctx->mix, 3 * sizeof(double), hipMemcpyDeviceToHost,
-                              s));
         HIPCHK(hipStreamSynchronize(s));
         prof_harvest(ctx);
         rel = std::sqrt(ctx->mix_h[1]) / std::sqrt(ctx->mix_h[0]);

@@ -177,7 +177,8 @@ template <typename T>
 void launch_pb_update_xr(const Geo &g, hipStream_t s, int first, const double *part_in,
                          const T *ph, const T *sh, const T *sv, const T *t, const T *r0,
                          double *e, T *r, double *part_out, PBState *st);
-void launch_pb_end(const Geo &g, hipStream_t s, const double *part, PBState *st);
+// host: pinned, takes the state as the kernel leaves it
+void launch_pb_end(const Geo &g, hipStream_t s, const double *part, PBState *st, PBState *host);
 
 // iterative refinement: the FP64 residual into r, r0 (the correction e, FP64 in both
 // modes, starts at 0 through the inner solve's first update), x += e with x kept in xb,
@@ -186,6 +187,7 @@ template <typename T>
 void launch_mixed_resid(const Geo &g, hipStream_t s, int pre, const double *b, const double *x,
                         T *r, T *r0, double *part);
 void launch_mixed_update(const Geo &g, hipStream_t s, double *x, const double *e, double *xb);
+// out: three sums, pinned host memory
 void launch_mixed_fold(const Geo &g, hipStream_t s, const double *part, double *out);
 
 void launch_bicg_fin0(const Geo &g, hipStream_t s, double *part, KState *st);

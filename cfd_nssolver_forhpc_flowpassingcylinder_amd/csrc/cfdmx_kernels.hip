@@ -1598,7 +1598,7 @@ __global__ void __launch_bounds__(kThreads)
 k_mixed_fold(const double *part, int nb, double *out)
 {
     double t[3];
-    fold_partials<3>(part, nb, nb, t);
+    fold_partials<3, kFoldAlone>(part, nb, nb, t);
     if (threadIdx.x == 0) {
         out[0] = t[0];
         out[1] = t[1];

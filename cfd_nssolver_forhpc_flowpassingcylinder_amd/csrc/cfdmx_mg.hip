@@ -123,7 +123,8 @@ __global__ void __launch_bounds__(256) k_mg_prolong(MGLevelT<T> F, MGLevelT<T> C
 }
 
 // coarse right-hand side: mean over the children of the fine residual f - A u
-template <typename T>
+// (LDS: their loads need no overlap, and absent children are left out)
+template <bool LDS = false, typename T>
 __device__ __forceinline__ void mg_restrict_at(const MGLevelT<T> &F, const MGLevelT<T> &C, int m)
 {
     int I, J, K;
@@ -137,6 +138,7 @@ __device__ __forceinline__ void mg_restrict_at(const MGLevelT<T> &F, const MGLev
     for (int q = 0; q < 8; ++q) {
         const int a = q >> 2, b = (q >> 1) & 1, c = q & 1;
         const bool ok = a < C.fx && b < C.fy && c < C.fz;
+        if (LDS && !ok) continue;
         const int i = I * C.fx + (ok ? a : 0), j = J * C.fy + (ok ? b : 0),
                   k = K * C.fz + (ok ? c : 0);
         const int n = (i * F.ny + j) * F.nz + k;
@@ -249,36 +251,37 @@ struct MGTail {
     int nlev;
 };
 
-// half sweep of colour c over a level in LDS
+// half sweep of colour c over a level in LDS.  The threads count cells of the colour: nz / 2 of
+// each row (below the top plane where nz is odd), then every other row's cell of that plane.
+// Counted over all cells, with half of the threads idle, k_mg_tail took 37.7 us for 48x24x3 and
+// below in FP32, now 28.1: the instructions of one CU bound it, 0.4 us for 1024 cells.
 template <typename T>
 __device__ __forceinline__ void mg_tail_sweep(const MGLevelT<T> &L, int c)
 {
     const int tid = threadIdx.x, nt = blockDim.x;
     const T *u = L.u;
-    auto cell = [&](int n, int i, int j, int k) {
+    auto cell = [&](int row, int i, int j, int k) {
+        const int n = row * L.nz + k;
         const T s = mg_nbsum(L, n, i, j, k, [&](int q, int, int, int) { return u[q]; });
         L.u[n] = (L.f[n] + s) / mg_diag(L, i, j, k);
     };
-    if ((L.nz & 1) == 0) {
-        const int half = L.nz >> 1;
-        for (int m = tid; m < (L.n >> 1); m += nt) {
-            const int row = (int)fdiv((unsigned)m, L.dzh);
-            const int i = (int)fdiv((unsigned)row, L.dy), j = row - i * L.ny;
-            const int k = 2 * (m - row * half) + ((i + j + c) & 1);
-            cell(row * L.nz + k, i, j, k);
-        }
-    } else {
+    const int half = L.nz >> 1, rows = L.nx * L.ny;
+    for (int m = tid; m < rows * half; m += nt) {
+        const int row = (int)fdiv((unsigned)m, L.dzh);
+        const int i = (int)fdiv((unsigned)row, L.dy), j = row - i * L.ny;
+        cell(row, i, j, 2 * (m - row * half) + ((i + j + c) & 1));
+    }
+    if (L.nz & 1) {
         // periodic z joins two cells of one colour: their planes in turn (k_mg_smooth_cell)
-        const bool wrap_same = L.zper && L.nz > 1;
-        for (int pass = 0; pass < (wrap_same ? 2 : 1); ++pass) {
-            if (pass) __syncthreads();
-            for (int n = tid; n < L.n; n += nt) {
-                int i, j, k;
-                mg_coords(L, n, i, j, k);
-                if (((i + j + k) & 1) != c) continue;
-                if (wrap_same && (k == L.nz - 1) != (pass == 1)) continue;
-                cell(n, i, j, k);
-            }
+        if (L.zper && L.nz > 1) __syncthreads();
+        const int top = L.nz - 1; // even: the colour's rows are those of i + j of c's parity
+        for (int m = tid; m < (rows + 1) >> 1; m += nt) {
+            int row = 2 * m, i = (int)fdiv((unsigned)row, L.dy);
+            // i + j runs with the row number where ny is odd; else row 2m and the next share i
+            row += L.ny & 1 ? c : (i + c) & 1;
+            if (row >= rows) continue;
+            i = (int)fdiv((unsigned)row, L.dy);
+            cell(row, i, row - i * L.ny, top);
         }
     }
     __syncthreads();
@@ -313,7 +316,7 @@ __global__ void __launch_bounds__(kMGCoarseThreads) k_mg_tail(MGTail<T> t)
         mg_tail_sweep(F, 1);
         mg_tail_sweep(F, 0);
         mg_tail_sweep(F, 1);
-        for (int m = tid; m < C.n; m += nt) mg_restrict_at(F, C, m);
+        for (int m = tid; m < C.n; m += nt) mg_restrict_at<true>(F, C, m);
         __syncthreads();
     }
     {
@@ -489,30 +492,55 @@ __global__ void k_pb_update_p(Geo g, int first, const T *r, const T *v, T *p, co
         p[n] = first ? r[n] : r[n] + beta * (p[n] - om * v[n]);
 }
 
-// alpha = rho / (v, r0) (one workgroup)
+// Up to this many partials every block of the kernel that uses a scalar folds them itself
+// (a block and all of them in flight together: 1 to 2 us); above, a kernel of one block does
+// it once.  A solve's iteration at 96x48x6 (27 partials) and 256x128x32 (1024) measured
+// 8 and 6 us less so; at 512x256x64 (8192) each block would read 64 KiB.
+constexpr int kPBFoldEach = 1024;
+// alpha = rho / (v, r0)
+template <int U>
+__device__ __forceinline__ double pb_alpha(const Geo &g, const double *part, const PBState *st)
+{
+    double t[1];
+    fold_partials<1, U>(part, g.nblocks, g.nblocks, t);
+    return st->rho / t[0];
+}
 __global__ void __launch_bounds__(kThreads) k_pb_alpha(Geo g, const double *part, PBState *st)
 {
     if (st->done) return;
-    double t[1];
-    fold_partials<1>(part, g.nblocks, g.nblocks, t);
-    if (threadIdx.x == 0) st->alpha = st->rho / t[0];
+    const double alpha = pb_alpha<kFoldAlone>(g, part, st);
+    if (threadIdx.x == 0) st->alpha = alpha;
 }
 
-// omega = (t, s) / (t, t) (one workgroup)
+// omega = (t, s) / (t, t)
+template <int U>
+__device__ __forceinline__ double pb_omega(const Geo &g, const double *part)
+{
+    double t[2];
+    fold_partials<2, U>(part, g.nblocks, g.nblocks, t);
+    return t[0] / t[1];
+}
 __global__ void __launch_bounds__(kThreads) k_pb_omega(Geo g, const double *part, PBState *st)
 {
     if (st->done) return;
-    double t[2];
-    fold_partials<2>(part, g.nblocks, g.nblocks, t);
-    if (threadIdx.x == 0) st->omega = t[0] / t[1];
+    const double omega = pb_omega<kFoldAlone>(g, part);
+    if (threadIdx.x == 0) st->omega = omega;
 }
 
-// s = r - alpha v
-template <typename T>
-__global__ void k_pb_update_s(Geo g, const T *r, const T *v, T *s, const PBState *st)
+// s = r - alpha v; FOLD: alpha from the partials of (v, r0), for the kernels to come too
+template <typename T, bool FOLD>
+__global__ void __launch_bounds__(kThreads)
+k_pb_update_s(Geo g, const double *part, const T *r, const T *v, T *s, PBState *st)
 {
     if (st->done) return;
-    const T a = (T)st->alpha;
+    double alpha;
+    if constexpr (FOLD) {
+        alpha = pb_alpha<8>(g, part, st);
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->alpha = alpha;
+    } else {
+        alpha = st->alpha;
+    }
+    const T a = (T)alpha;
     for (int n = blockIdx.x * blockDim.x + threadIdx.x; n < g.N; n += gridDim.x * blockDim.x)
         s[n] = r[n] - a * v[n];
 }
@@ -524,38 +552,55 @@ __global__ void k_pb_update_s(Geo g, const T *r, const T *v, T *s, const PBState
 // the FP32 recursion's drift from the true residual, ~1e-6.  FIRST (the solve's first
 // iteration, e = 0): e is written as +0.0 plus the increment without being read, which is
 // the sum the zeroed vector would give, -0.0 turning to +0.0 included.
-template <typename T, bool FIRST>
+// FOLD: omega from the partials of (t, s), (t, t).
+template <typename T, bool FIRST, bool FOLD>
 __global__ void __launch_bounds__(kThreads)
-k_pb_update_xr(Geo g, const T *ph, const T *sh, const T *s, const T *t, const T *r0, double *e,
-               T *r, double *part_out, const PBState *st)
+k_pb_update_xr(Geo g, const double *part_in, const T *__restrict__ ph, const T *__restrict__ sh,
+               const T *__restrict__ s, const T *__restrict__ t, const T *__restrict__ r0,
+               double *__restrict__ e, T *__restrict__ r, double *part_out, PBState *st)
 {
     if (st->done) return;
     const int B = logical_block(g);
     if (B >= g.nblocks) return;
-    const T om = (T)st->omega;
-    const double ad = st->alpha, omd = st->omega;
+    const double ad = st->alpha;
+    double omd;
+    if constexpr (FOLD) {
+        omd = pb_omega<8>(g, part_in);
+        if (B == 0 && threadIdx.x == 0) st->omega = omd;
+    } else {
+        omd = st->omega;
+    }
+    const T om = (T)omd;
     double acc[2] = {0.0, 0.0};
-    for (int c = 0; c < kCells; ++c) {
-        const int n = B * kPerBlock + c * kThreads + threadIdx.x;
-        if (n < g.N) {
-            const double inc = ad * (double)ph[n] + omd * (double)sh[n];
-            if constexpr (FIRST) e[n] = 0.0 + inc;
-            else e[n] += inc;
-            const T rn = s[n] - om * t[n];
-            r[n] = rn;
-            acc[0] += (double)rn * (double)rn;
-            acc[1] += (double)rn * (double)r0[n];
+    auto cell = [&](int n) {
+        const double inc = ad * (double)ph[n] + omd * (double)sh[n];
+        if constexpr (FIRST) e[n] = 0.0 + inc;
+        else e[n] += inc;
+        const T rn = s[n] - om * t[n];
+        r[n] = rn;
+        acc[0] += (double)rn * (double)rn;
+        acc[1] += (double)rn * (double)r0[n];
+    };
+    if ((B + 1) * kPerBlock <= g.N) {
+#pragma unroll
+        for (int c = 0; c < kCells; ++c) cell(B * kPerBlock + c * kThreads + threadIdx.x);
+    } else {
+        for (int c = 0; c < kCells; ++c) {
+            const int n = B * kPerBlock + c * kThreads + threadIdx.x;
+            if (n < g.N) cell(n);
         }
     }
     block_sums<2>(acc, part_out, g.nblocks, B);
 }
 
-// end of an iteration: residual test, rho and beta for the next one
-__global__ void __launch_bounds__(kThreads) k_pb_end(Geo g, const double *part, PBState *st)
+// end of an iteration: residual test, rho and beta for the next one.  host: the host's copy of
+// the state in pinned memory, written here (a copy after the kernel is a kernel of its own)
+__global__ void __launch_bounds__(kThreads)
+k_pb_end(Geo g, const double *part, PBState *st, PBState *host)
 {
     if (st->done) return;
     double t[2];
-    fold_partials<2>(part, g.nblocks, g.nblocks, t);
+    fold_partials<2, kFoldAlone>(part, g.nblocks, g.nblocks, t);
     if (threadIdx.x == 0) {
         const double res = sqrt(t[0]) / st->norm0;
         st->res = res;
@@ -565,6 +610,7 @@ __global__ void __launch_bounds__(kThreads) k_pb_end(Geo g, const double *part, 
         st->rho = rho;
         if (res < st->tol) st->done = 1;
         else if (st->iter >= st->maxit || !(res == res)) st->done = 2;
+        *host = *st;
     }
 }
 
@@ -797,16 +843,22 @@ template <typename T>
 void launch_pb_update_p(const Geo &g, hipStream_t s, int first, const T *r, const T *v, T *p,
                         const PBState *st)
 {
-    hipLaunchKernelGGL(k_pb_update_p<T>, dim3(2048), dim3(256), 0, s, g, first, r, v, p, st);
+    hipLaunchKernelGGL(k_pb_update_p<T>, dim3(std::min(2048, cdiv(g.N, 256))), dim3(256), 0, s, g,
+                       first, r, v, p, st);
 }
 
 template <typename T>
 void launch_pb_update_s(const Geo &g, hipStream_t s, const double *part, const T *r, const T *v,
                         T *sv, PBState *st)
 {
+    if (g.nblocks <= kPBFoldEach) {
+        hipLaunchKernelGGL((k_pb_update_s<T, true>), dim3(std::min(2048, cdiv(g.N, kThreads))),
+                           dim3(kThreads), 0, s, g, part, r, v, sv, st);
+        return;
+    }
     hipLaunchKernelGGL(k_pb_alpha, dim3(1), dim3(kThreads), 0, s, g, part, st);
-    hipLaunchKernelGGL(k_pb_update_s<T>, dim3(2048), dim3(256), 0, s, g, r, v, sv,
-                       (const PBState *)st);
+    hipLaunchKernelGGL((k_pb_update_s<T, false>), dim3(2048), dim3(kThreads), 0, s, g, part, r, v,
+                       sv, st);
 }
 
 template <typename T>
@@ -814,18 +866,19 @@ void launch_pb_update_xr(const Geo &g, hipStream_t s, int first, const double *p
                          const T *ph, const T *sh, const T *sv, const T *t, const T *r0,
                          double *e, T *r, double *part_out, PBState *st)
 {
-    hipLaunchKernelGGL(k_pb_omega, dim3(1), dim3(kThreads), 0, s, g, part_in, st);
-    if (first)
-        hipLaunchKernelGGL((k_pb_update_xr<T, true>), dim3(lin_blocks(g)), dim3(kThreads), 0, s,
-                           g, ph, sh, sv, t, r0, e, r, part_out, (const PBState *)st);
-    else
-        hipLaunchKernelGGL((k_pb_update_xr<T, false>), dim3(lin_blocks(g)), dim3(kThreads), 0, s,
-                           g, ph, sh, sv, t, r0, e, r, part_out, (const PBState *)st);
+    const bool fold = g.nblocks <= kPBFoldEach;
+    if (!fold) hipLaunchKernelGGL(k_pb_omega, dim3(1), dim3(kThreads), 0, s, g, part_in, st);
+    auto run = [&](auto k) {
+        hipLaunchKernelGGL(k, dim3(lin_blocks(g)), dim3(kThreads), 0, s, g, part_in, ph, sh, sv,
+                           t, r0, e, r, part_out, st);
+    };
+    if (first) run(fold ? k_pb_update_xr<T, true, true> : k_pb_update_xr<T, true, false>);
+    else run(fold ? k_pb_update_xr<T, false, true> : k_pb_update_xr<T, false, false>);
 }
 
-void launch_pb_end(const Geo &g, hipStream_t s, const double *part, PBState *st)
+void launch_pb_end(const Geo &g, hipStream_t s, const double *part, PBState *st, PBState *host)
 {
-    hipLaunchKernelGGL(k_pb_end, dim3(1), dim3(kThreads), 0, s, g, part, st);
+    hipLaunchKernelGGL(k_pb_end, dim3(1), dim3(kThreads), 0, s, g, part, st, host);
 }
 
 #define CFDMX_MG_INSTANCES(T)                                                                 \
