@@ -622,7 +622,15 @@ static int setup_device(cfdmx_ctx *ctx)
     g.cd_tj = kThreads / g.cd_tk;
     g.cd_nkt = (g.nzc + g.cd_tk - 1) / g.cd_tk;
     g.cd_njt = (g.nyc + g.cd_tj - 1) / g.cd_tj;
-    g.cd_nb = g.cd_nkt * g.cd_njt * g.nchunk;
+    // The longest march of planes with more than two blocks a CU (256 CUs), else one plane a
+    // block: a long march reads two planes of halo less often, a short one fills the chip.  8,
+    // 4, 2, 1 planes: 96x48x6 (2 tiles) 35, 21, 14.7, 11.5 us; 128x128x16 (8) 32.8, 21.1,
+    // 17.6, 18.0; 197x93x31 (12) 43.4, 33.0, 34.3, 42.6; 256x128x32 (16) 41.6, 36.8, 43.4,
+    // 56.5; 300x160x40 (40) 96.6, 109, 133, 175.
+    g.cd_ch = kChunk;
+    auto cd_blocks = [&] { return g.cd_nkt * g.cd_njt * ((c.nx + g.cd_ch - 1) / g.cd_ch); };
+    while (g.cd_ch > 1 && cd_blocks() <= 512) g.cd_ch /= 2;
+    g.cd_nb = cd_blocks();
 
     // metric tables in one buffer
     std::vector<double> buf;

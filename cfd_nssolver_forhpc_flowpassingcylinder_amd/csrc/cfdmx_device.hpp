@@ -100,8 +100,9 @@ struct Geo {
     FastDiv dz, dy;    // by nzc, by nyc
     int ntile, nchunk, nmarch; // plane tiles, plane chunks, march blocks
     // conv-diff tiles: cd_tk cells of k by cd_tj rows of j (cd_tk * cd_tj = 256), tiles
-    // along k and j, blocks (tiles x plane chunks); the CFL partials are per block
-    int cd_tk, cd_tj, cd_nkt, cd_njt, cd_nb;
+    // along k and j, planes a block marches over, blocks (tiles x marches); the CFL partials
+    // are per block
+    int cd_tk, cd_tj, cd_nkt, cd_njt, cd_ch, cd_nb;
     Axis ax[3];
     PAxis pa[3];
 };

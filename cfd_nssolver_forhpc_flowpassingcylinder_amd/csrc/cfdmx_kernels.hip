@@ -103,7 +103,7 @@ __device__ __forceinline__ void load5(const double *phi, int c, int s, double f[
 //
 // Plane-marching and LDS-tiled: a block owns a tile of TJ rows x TK cells of the (j, k)
 // plane (TK the power of two >= nzc, 4 to 32; TJ = 256 / TK; one cell per thread)
-// and marches over kChunk planes in x.  A 3-slot LDS ring holds u, v, w of the planes
+// and marches over cd_ch planes in x.  A 3-slot LDS ring holds u, v, w of the planes
 // behind, at and ahead of the current one over the tile plus two rows and two cells of
 // halo on each side (the y and z stencils and the cross terms); the thread's own column
 // at two planes behind and ahead (the rest of the x stencil) stays in registers.  The
@@ -143,7 +143,7 @@ __device__ __forceinline__ Axis cd_axis_lds(const Axis &a, int lo, int n, int li
 __host__ __device__ inline size_t cd_lds_bytes(const Geo &g)
 {
     const size_t P = (size_t)(g.cd_tj + 4) * (g.cd_tk + 4);
-    return (9 * P + kCdTables * ((size_t)(kChunk + 4) + (g.cd_tj + 4) + (g.cd_tk + 4))) *
+    return (9 * P + kCdTables * ((size_t)(g.cd_ch + 4) + (g.cd_tj + 4) + (g.cd_tk + 4))) *
            sizeof(double);
 }
 
@@ -161,14 +161,14 @@ k_convdiff(Geo g, const double *__restrict__ u, const double *__restrict__ v,
     extern __shared__ double lds[];
     const int TK = g.cd_tk, TJ = g.cd_tj, RW = TK + 4, P = (TJ + 4) * RW;
     const int kt = b % g.cd_nkt, jt = (b / g.cd_nkt) % g.cd_njt, ch = b / (g.cd_nkt * g.cd_njt);
-    const int k0 = kt * TK, j0 = jt * TJ, i0 = ch * kChunk;
-    const int I0 = i0 + kGC, len = min(kChunk, g.nxc - i0);
+    const int k0 = kt * TK, j0 = jt * TJ, i0 = ch * g.cd_ch;
+    const int I0 = i0 + kGC, len = min(g.cd_ch, g.nxc - i0);
     double *ring = lds;                 // [slot][field][P]
     double *mt = lds + 9 * P;           // metric tables
-    const Axis X = cd_axis_lds(g.ax[0], I0 - 2, kChunk + 4, g.nx, mt);
-    const Axis Y = cd_axis_lds(g.ax[1], j0, TJ + 4, g.ny, mt + kCdTables * (kChunk + 4));
+    const Axis X = cd_axis_lds(g.ax[0], I0 - 2, g.cd_ch + 4, g.nx, mt);
+    const Axis Y = cd_axis_lds(g.ax[1], j0, TJ + 4, g.ny, mt + kCdTables * (g.cd_ch + 4));
     const Axis Z = cd_axis_lds(g.ax[2], k0, TK + 4,
-                               g.nz, mt + kCdTables * (kChunk + 4 + TJ + 4));
+                               g.nz, mt + kCdTables * (g.cd_ch + 4 + TJ + 4));
     // own cell
     const int tj = threadIdx.x / TK, tk = threadIdx.x - tj * TK;
     const int J = j0 + tj + kGC, K = k0 + tk + kGC;
