@@ -601,11 +601,18 @@ __global__ void k_bc_y(Geo g, BCParams bc, double *u, double *v, double *w, doub
     p[e1] = pn;
 }
 
-__global__ void k_bc_z(Geo g, BCParams bc, double *u, double *v, double *w, double *p,
-                       double *u1, double *v1, double *w1)
+// One thread a column and field (blockIdx.y: u, v, w, p), what it copies read before the first
+// store.  The columns' ends are lines apart: latency bounds small grids (96x48x6: 6.7 us with all
+// fields in one thread, each after the stores of the one before, now 3.6; 384x192x48 22.7 and
+// 20.8), whole lines for 16 bytes of each the large ones (512x256x64 44 and 45 us).
+__global__ void __launch_bounds__(kThreads)
+k_bc_z(Geo g, BCParams bc, double *u, double *v, double *w, double *p, double *u1, double *v1,
+       double *w1)
 {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    const int m = blockIdx.x * blockDim.x + threadIdx.x, q = blockIdx.y;
     const int nz = g.nz, nzc = g.nzc;
+    double *f = q == 0 ? u : q == 1 ? v : q == 2 ? w : p;
+    double *f1 = q == 0 ? u1 : q == 1 ? v1 : q == 2 ? w1 : nullptr;
     if (g.zper) {
         // periodic: ghost k <- k + nzc (k < 2) or k - nzc (k >= nz-2) for u, v, w and p
         // in every (i,j) column (the face k = nz-3 reads x/y ghost columns); T1 receives
@@ -614,101 +621,75 @@ __global__ void k_bc_z(Geo g, BCParams bc, double *u, double *v, double *w, doub
         const int I = m / g.ny, J = m % g.ny;
         const int b = gidx(g, I, J, 0);
         const bool inner = I >= kGC && I < g.nx - kGC && J >= kGC && J < g.ny - kGC;
-        double *f[4] = {u, v, w, p};
-        double *f1[4] = {u1, v1, w1, nullptr};
-        for (int q = 0; q < 4; ++q) {
-            const double a1 = f[q][b + 1 + nzc], a0 = f[q][b + nzc];
-            const double a2 = f[q][b + nz - 2 - nzc], a3 = f[q][b + nz - 1 - nzc];
-            f[q][b + 1] = a1;
-            f[q][b + 0] = a0;
-            f[q][b + nz - 2] = a2;
-            f[q][b + nz - 1] = a3;
-            if (f1[q] && inner) {
-                f1[q][b + 1] = a1;
-                f1[q][b + 0] = a0;
-                f1[q][b + nz - 2] = a2;
-                f1[q][b + nz - 1] = a3;
-                if (q == 2) f1[q][b + nz - 3] = f[q][b + nz - 3];
-            }
+        const double a1 = f[b + 1 + nzc], a0 = f[b + nzc];
+        const double a2 = f[b + nz - 2 - nzc], a3 = f[b + nz - 1 - nzc];
+        f[b + 1] = a1;
+        f[b + 0] = a0;
+        f[b + nz - 2] = a2;
+        f[b + nz - 1] = a3;
+        if (f1 && inner) {
+            f1[b + 1] = a1;
+            f1[b + 0] = a0;
+            f1[b + nz - 2] = a2;
+            f1[b + nz - 1] = a3;
+            if (q == 2) f1[b + nz - 3] = a1; // k = nz - 3 = 1 + nzc
         }
         return;
     }
     if (m >= g.nxc * g.nyc) return;
     const int I = m / g.nyc + kGC, J = m % g.nyc + kGC;
     const int b = gidx(g, I, J, 0);
-    // face 4 (:121-129)
-    put2(u, u1, b + 1, b, bc.dir[4][0] * 2. + (2.0 * bc.num[4][0] - 1.0) * u[b + 2]);
-    put2(v, v1, b + 1, b, bc.dir[4][1] * 2. + (2.0 * bc.num[4][1] - 1.0) * v[b + 2]);
-    put2(w, w1, b + 1, b, bc.dir[4][2] + bc.num[4][2] * w[b + 2]);
-    // face 5 (:133-143)
-    const double wb = bc.dir[5][2] + bc.num[5][2] * w[b + nz - 4];
-    w[b + nz - 1] = wb;
-    w[b + nz - 2] = wb;
-    w[b + nz - 3] = wb;
-    if (w1) {
-        w1[b + nz - 1] = wb;
-        w1[b + nz - 2] = wb;
-        w1[b + nz - 3] = wb;
+    const double lo = f[b + 2], hi = f[b + nz - (q == 2 ? 4 : 3)];
+    if (q == 2) {
+        // face 4 (:121-129), face 5 (:133-143): w has its own
+        put2(f, f1, b + 1, b, bc.dir[4][2] + bc.num[4][2] * lo);
+        const double wb = bc.dir[5][2] + bc.num[5][2] * hi;
+        put2(f, f1, b + nz - 1, b + nz - 2, wb);
+        f[b + nz - 3] = wb;
+        if (f1) f1[b + nz - 3] = wb;
+    } else if (q == 3) {
+        // pressure (:166-172)
+        put2(f, nullptr, b + 1, b, lo);
+        put2(f, nullptr, b + nz - 2, b + nz - 1, hi);
+    } else {
+        put2(f, f1, b + 1, b, bc.dir[4][q] * 2. + (2.0 * bc.num[4][q] - 1.0) * lo);
+        put2(f, f1, b + nz - 2, b + nz - 1,
+             bc.dir[5][q] * 2. + (2.0 * bc.num[5][q] - 1.0) * hi);
     }
-    put2(u, u1, b + nz - 2, b + nz - 1,
-         bc.dir[5][0] * 2. + (2.0 * bc.num[5][0] - 1.0) * u[b + nz - 3]);
-    put2(v, v1, b + nz - 2, b + nz - 1,
-         bc.dir[5][1] * 2. + (2.0 * bc.num[5][1] - 1.0) * v[b + nz - 3]);
-    // pressure (:166-172)
-    const double pb = p[b + 2];
-    p[b + 1] = pb;
-    p[b + 0] = pb;
-    const double pt = p[b + nz - 3];
-    p[b + nz - 2] = pt;
-    p[b + nz - 1] = pt;
 }
 
-// BC_staggered_copy (updateBC.hpp:6-110) on its own: ghost entries T0 -> T1
-__global__ void k_bc_copy(Geo g, const double *u0, const double *v0, const double *w0,
-                          double *u1, double *v1, double *w1)
+// BC_staggered_copy (updateBC.hpp:6-110) on its own: ghost entries T0 -> T1, one thread a
+// column of an axis and component (384x192x48: 30.4 us with all three in one thread, now 14.2)
+__global__ void __launch_bounds__(kThreads)
+k_bc_copy(Geo g, const double *u0, const double *v0, const double *w0, double *u1, double *v1,
+          double *w1)
 {
     int m = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nx = g.nx, ny = g.ny, nz = g.nz;
+    const int q = blockIdx.y;
+    const double *__restrict__ f0 = q == 0 ? u0 : q == 1 ? v0 : w0;
+    double *__restrict__ f1 = q == 0 ? u1 : q == 1 ? v1 : w1;
+    // along axis a, from a column's first entry: entries 0, 1, n - 2, n - 1 and, for the axis's
+    // own component, n - 3
+    const auto copy = [&](int a, int b, int stride, int n) {
+        const double x0 = f0[b], x1 = f0[b + stride], x2 = f0[b + (n - 3) * stride],
+                     x3 = f0[b + (n - 2) * stride], x4 = f0[b + (n - 1) * stride];
+        f1[b] = x0;
+        f1[b + stride] = x1;
+        if (q == a) f1[b + (n - 3) * stride] = x2;
+        f1[b + (n - 2) * stride] = x3;
+        f1[b + (n - 1) * stride] = x4;
+    };
     if (m < g.cyz) {
-        const int J = m / g.nzc + kGC, K = m % g.nzc + kGC;
-        const int cs[5] = {0, 1, nx - 3, nx - 2, nx - 1};
-        for (int q = 0; q < 5; ++q) {
-            const int c = gidx(g, cs[q], J, K);
-            u1[c] = u0[c];
-            if (q != 2) {
-                v1[c] = v0[c];
-                w1[c] = w0[c];
-            }
-        }
+        copy(0, gidx(g, 0, m / g.nzc + kGC, m % g.nzc + kGC), g.sx, g.nx);
         return;
     }
     m -= g.cyz;
     if (m < g.nxc * g.nzc) {
-        const int I = m / g.nzc + kGC, K = m % g.nzc + kGC;
-        const int cs[5] = {0, 1, ny - 3, ny - 2, ny - 1};
-        for (int q = 0; q < 5; ++q) {
-            const int c = gidx(g, I, cs[q], K);
-            v1[c] = v0[c];
-            if (q != 2) {
-                u1[c] = u0[c];
-                w1[c] = w0[c];
-            }
-        }
+        copy(1, gidx(g, m / g.nzc + kGC, 0, m % g.nzc + kGC), g.sy, g.ny);
         return;
     }
     m -= g.nxc * g.nzc;
-    if (m < g.nxc * g.nyc) {
-        const int I = m / g.nyc + kGC, J = m % g.nyc + kGC;
-        const int cs[5] = {0, 1, nz - 3, nz - 2, nz - 1};
-        for (int q = 0; q < 5; ++q) {
-            const int c = gidx(g, I, J, cs[q]);
-            w1[c] = w0[c];
-            if (q != 2) {
-                u1[c] = u0[c];
-                v1[c] = v0[c];
-            }
-        }
-    }
+    if (m < g.nxc * g.nyc) copy(2, gidx(g, m / g.nyc + kGC, m % g.nyc + kGC, 0), 1, g.nz);
 }
 
 // ---------------------------------------------------------------------------
@@ -2494,16 +2475,16 @@ void launch_bc(const Geo &g, hipStream_t s, const BCParams &bc, int advance, dou
     hipLaunchKernelGGL(k_bc_y, dim3(cdiv(g.nxc * g.nzc, 256)), dim3(256), 0, s, g, bc, u, v, w,
                        p, u1, v1, w1);
     const int nzcols = g.zper ? g.nx * g.ny : g.nxc * g.nyc;
-    hipLaunchKernelGGL(k_bc_z, dim3(cdiv(nzcols, 256)), dim3(256), 0, s, g, bc, u, v, w, p, u1,
-                       v1, w1);
+    hipLaunchKernelGGL(k_bc_z, dim3(cdiv(nzcols, kThreads), 4), dim3(kThreads), 0, s, g, bc, u, v,
+                       w, p, u1, v1, w1);
 }
 
 void launch_bc_copy(const Geo &g, hipStream_t s, const double *u0, const double *v0,
                     const double *w0, double *u1, double *v1, double *w1)
 {
     const int tot = g.cyz + g.nxc * g.nzc + g.nxc * g.nyc;
-    hipLaunchKernelGGL(k_bc_copy, dim3(cdiv(tot, 256)), dim3(256), 0, s, g, u0, v0, w0, u1, v1,
-                       w1);
+    hipLaunchKernelGGL(k_bc_copy, dim3(cdiv(tot, kThreads), 3), dim3(kThreads), 0, s, g, u0, v0, w0,
+                       u1, v1, w1);
 }
 
 void launch_rhs(const Geo &g, hipStream_t s, int pre, const double *us, const double *vs,
