@@ -45,7 +45,7 @@ BYTES_PER_CELL = {
     "convdiff": 48,  # r u, v, w;  w u*, v*, w*
     "rhs": 32,       # r u*, v*, w*;  w b
     "project": 96,   # r u*, v*, w*, X, eta;  w u, v, w, p, f(3)
-    "sor_half": 16,  # colour-split half sweep: r p (other colour), p, rhs (own);  w p (own)
+    "sor_half": 24,  # pass of two red-black sweeps: r p, rhs;  w p
 }
 
 # the BiCGSTAB iteration (phases A + B + C) is the FP64 step's dominant work: 128 B/cell
@@ -603,7 +603,7 @@ def rbsor_run(wl, args):
     """The metric's grid with the second pressure solver: red-black SOR on SorPipeLine's
     coefficients (omega 1.8, tol 1e-10 on max |dp| per sweep), sweeps per step capped at
     args.sor_maxit (the reference's p_sor_iter_max is 5000).  W warm-up and K timed steps
-    (wall clock), then one profiled step for the half-sweep kernel's rate."""
+    (wall clock), then one profiled step for the rate of the pass of two sweeps."""
     s = make_solver(wl, "none", "rbsor", args.seed, args.sor_maxit, 0)
     for q in range(args.warmup):
         s.step(1)
@@ -632,20 +632,21 @@ def rbsor_run(wl, args):
         "ms_per_step": round(wall / args.steps * 1e3, 3),
         "config": (f"{wl['nx']}x{wl['ny']}x{wl['nz']}, Re={wl['re']:g}, dt={wl['dt']:g}, "
                    f"red-black SOR omega 1.8, tol {wl['tol']:g} (max |dp| per sweep), at most "
-                   f"{args.sor_maxit} sweeps per step, FP64, colour-split storage"),
+                   f"{args.sor_maxit} sweeps per step, FP64, two sweeps a pass"),
         "sweep_cap": args.sor_maxit,
         "sweeps_per_step": sweeps, "max_dp_per_step": [i["err"] for i in infos],
         "steps_reaching_tol": sum(1 for i in infos if i["err"] < wl["tol"]),
         "ms_per_sweep": round(wall / sum(sweeps) * 1e3, 4),
-        "roofline": {"bound": "hbm", "kernel": "k_sor_rb2 (one colour's half sweep)",
+        "roofline": {"bound": "hbm", "kernel": "k_sor_pass (two sweeps)",
                      "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": measured_traffic(args.workload, "sor_half"),
+                     "traffic": measured_traffic(args.workload, "sor_pass"),
                      "avg_launch_us": round(avg_s * 1e6, 2),
                      "bytes_per_launch": BYTES_PER_CELL["sor_half"] * n_cells,
-                     "bytes_note": ("16 B per cell of the grid per half sweep: the other "
-                                    "colour read, own p and right-hand side read, own p "
-                                    "written (32 B/cell per full sweep)")},
+                     "bytes_note": ("24 B per cell of the grid per pass: p and the "
+                                    "right-hand side read, p written (12 B/cell per full "
+                                    "sweep); what blocks read twice around their tiles is "
+                                    "not counted")},
         "kernels": kernel_table(prof, n_cells, BYTES_PER_CELL),
     }
 

@@ -317,7 +317,7 @@ CFDMX_API int cfdmx_adjoint_drag(cfdmx_ctx *ctx, int nsteps, int checkpoint_ever
 #define CFDMX_K_BICG_B 5
 #define CFDMX_K_BICG_C 6
 #define CFDMX_K_BICG_CHECK 7 /* initial fold and end-of-batch convergence check */
-#define CFDMX_K_SOR 8
+#define CFDMX_K_SOR 8 /* a half sweep, or a pass of two sweeps where one kernel runs it */
 #define CFDMX_K_PROJECT 9
 #define CFDMX_K_MG 10 /* mixed precision: multigrid V-cycle kernels */
 #define CFDMX_K_PB 11 /* mixed precision: FP32 BiCGSTAB products and updates */
