@@ -1694,8 +1694,8 @@ static int solve_rbsor_passes(cfdmx_ctx *ctx)
         prof_harvest(ctx);
         if (ctx->sst_h->done) break;
     }
-    // the last pass read p or the copy as it was the ((iters - 1) / 2)-th or not; if its first
-    // sweep was the last one, that sweep alone is run again from there
+    // pass (iters - 1) / 2 was the last and read buf[from]; if it ended after its first sweep,
+    // that sweep alone is run again from there
     const int from = ((ctx->sst_h->iters - 1) / 2) & 1;
     if (ctx->sst_h->iters & 1) pass(from, {nullptr, nullptr, nullptr, part[0], 1});
     if (from == 0) launch_copy(s, g.G, buf[1], buf[0]);
