@@ -151,6 +151,7 @@ struct MGSweepT {
     int tz, pairs;                 // pairs of a row owned (half: whole rows) and held
     int njt, nkt, nblk;            // tiles in y and z, blocks
     T cx, cy, cz;
+    T tiny;                        // dividends below it are divided (mg_exactly)
     const T *f, *e;                // right-hand side; coarse correction (up)
     T *ub, *fc, *u;                // black half; coarse right-hand side (down); result (up)
 };

@@ -717,6 +717,9 @@ static MGSweepT<T> sweep_args(const MGLevelT<T> &F, const MGLevelT<T> &C)
     a.nx = F.nx, a.ny = F.ny, a.nz = F.nz, a.half = F.nz >> 1;
     a.fx = C.fx, a.fy = C.fy, a.fz = C.fz, a.cny = C.ny, a.cnz = C.nz;
     a.cx = F.cx, a.cy = F.cy, a.cz = F.cz;
+    // from here on a float dividend's quotient by any diagonal of the level is normal and the
+    // products that correct it are exact (2^-102)
+    a.tiny = std::max((T)0x1p-100, (T)0x1p-120 * (F.cx + F.cy + F.cz));
     a.f = F.f, a.e = C.u, a.ub = F.ub, a.fc = C.f, a.u = F.u;
     return a;
 }

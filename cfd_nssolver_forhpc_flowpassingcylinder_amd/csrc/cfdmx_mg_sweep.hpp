@@ -27,12 +27,15 @@
 #pragma once
 #include "cfdmx_internal.hpp"
 
+#include <type_traits>
+
 namespace cfdmx {
 
 constexpr int kMGHalo = 4;          // rows and planes a block forms again on each side
 constexpr int kMGSweepThreads = 512; // largest block of the sweep kernels
 
-// a / b from r = RN(1/b), correctly rounded (see divr); r = 0 gives 0
+// a / b from r = RN(1/b), correctly rounded (see divr) where the corrections' residuals and
+// the quotient have no subnormal part; r = 0 gives 0
 __device__ __forceinline__ double mg_quot(double a, double b, double r)
 {
     double q = a * r;
@@ -195,9 +198,10 @@ template <typename T, int P, bool ZPER> struct MGCol {
         return m;
     }
 
-    // (f + s) / d at pair q for a cell of parity PAR; d is returned too
-    template <int PAR>
-    __device__ __forceinline__ T quot(const MGDiag<T> &m, int q, T v, T &d) const
+    // (f + s) / d at pair q for a cell of parity PAR; d is returned too.  EXACT: by division;
+    // else `least` takes the magnitude of a dividend other than zero (as ordered bits, float)
+    template <int PAR, bool EXACT>
+    __device__ __forceinline__ T quot(const MGDiag<T> &m, int q, T v, T &d, unsigned &least) const
     {
         T r = m.r;
         d = m.d;
@@ -207,6 +211,9 @@ template <typename T, int P, bool ZPER> struct MGCol {
             r = miss ? rz : r;
             d = miss ? dz : d;
         }
+        if constexpr (EXACT) return r != (T)0 ? v / d : (T)0;
+        if constexpr (std::is_same<T, float>::value)
+            least = min(least, 2u * __float_as_uint(v) - 1u);
         return mg_quot(v, d, r);
     }
 
@@ -250,13 +257,26 @@ template <int V> struct MGInt {
 
 #define MG_INLINE __attribute__((always_inline))
 
+// A float dividend below a.tiny gives mg_quot a subnormal part.  A right-hand side of ordinary
+// size has none, so a block divides only in a second pass over its cells, if one of its threads
+// met such a dividend in the first; the results are then written again.  Steps of 24 grids took
+// 0 to 3% longer for looking at the dividends so, 3 to 11% with a branch at every quotient.  In
+// double such a value is 2^-400 times the largest of a residual whose norm does not underflow,
+// and is not looked for.
+template <typename T, class Pass>
+__device__ __forceinline__ void mg_exactly(const MGSweepT<T> &a, Pass &&pass)
+{
+    const unsigned least = pass(std::false_type());
+    if constexpr (std::is_same<T, float>::value)
+        if (__syncthreads_or(least < 2u * __float_as_uint(a.tiny) - 1u)) pass(std::true_type());
+}
+
 // GEN: 0 = z-only coarsening (fx = fy = 1, fz = 2); 1 = any other, by the factors in a
-template <typename T, int P, bool ZPER, int GEN>
-__global__ void __launch_bounds__(kMGSweepThreads) k_mg_down(MGSweepT<T> a)
+template <typename T, int P, bool ZPER, int GEN, bool EXACT>
+__device__ __forceinline__ unsigned mg_down(const MGSweepT<T> &a, const MGCol<T, P, ZPER> &c)
 {
     extern __shared__ double mg_lds[];
-    MGCol<T, P, ZPER> c;
-    if (!c.init(a)) return;
+    unsigned least = ~0u;
     const int SL = a.rows * mg_lds_row<P>(a.pairs);
     // half planes of the four half sweeps, two slots each: first red and black, second red
     // and black
@@ -304,7 +324,7 @@ __global__ void __launch_bounds__(kMGSweepThreads) k_mg_down(MGSweepT<T> a)
         T r1[P], x1[P];
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            r1[q] = c.template quot<PAR>(dg[S], q, fr[S][q], d);
+            r1[q] = c.template quot<PAR, EXACT>(dg[S], q, fr[S][q], d, least);
             x1[q] = a.cx * r1[q];
         }
         if (c.live) mg_put(L1 + e * SL + c.own, r1);
@@ -313,7 +333,7 @@ __global__ void __launch_bounds__(kMGSweepThreads) k_mg_down(MGSweepT<T> a)
         c.template sum<PAR>(a, L1 + o * SL, xr1[e], x1, r1m, s);
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            b1[q] = c.template quot<PAR>(dg[m1], q, fb[m1][q] + s[q], d);
+            b1[q] = c.template quot<PAR, EXACT>(dg[m1], q, fb[m1][q] + s[q], d, least);
             x2[q] = a.cx * b1[q];
             xr1[e][q] = x1[q];
             r1m[q] = r1[q];
@@ -324,7 +344,7 @@ __global__ void __launch_bounds__(kMGSweepThreads) k_mg_down(MGSweepT<T> a)
         c.template sum<PAR>(a, L2 + e * SL, xb1[o], x2, b1m, s);
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            r2[q] = c.template quot<PAR>(dg[m2], q, fr[m2][q] + s[q], d);
+            r2[q] = c.template quot<PAR, EXACT>(dg[m2], q, fr[m2][q] + s[q], d, least);
             x3[q] = a.cx * r2[q];
             xb1[o][q] = x2[q];
             b1m[q] = b1[q];
@@ -335,7 +355,7 @@ __global__ void __launch_bounds__(kMGSweepThreads) k_mg_down(MGSweepT<T> a)
         c.template sum<PAR>(a, L3 + o * SL, xr2[e], x3, r2m, s);
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            b2[q] = c.template quot<PAR>(dg[m3], q, fb[m3][q] + s[q], d);
+            b2[q] = c.template quot<PAR, EXACT>(dg[m3], q, fb[m3][q] + s[q], d, least);
             x4[q] = a.cx * b2[q];
             rbn[q] = fb[m3][q] - (d * b2[q] - s[q]);
             xr2[e][q] = x3[q];
@@ -436,15 +456,24 @@ __global__ void __launch_bounds__(kMGSweepThreads) k_mg_down(MGSweepT<T> a)
     // of barriers) on either side
     if (__builtin_amdgcn_readfirstlane(c.par0)) march(MGInt<1>());
     else march(MGInt<0>());
+    return least;
+}
+template <typename T, int P, bool ZPER, int GEN>
+__global__ void __launch_bounds__(kMGSweepThreads) k_mg_down(MGSweepT<T> a)
+{
+    MGCol<T, P, ZPER> c;
+    if (!c.init(a)) return;
+    mg_exactly(a, [&](auto exact) {
+        return mg_down<T, P, ZPER, GEN, decltype(exact)::value>(a, c);
+    });
 }
 
 // FZ2: the level was coarsened in z (a pair's cells have one parent)
-template <typename T, int P, bool ZPER, bool FZ2>
-__global__ void __launch_bounds__(kMGSweepThreads) k_mg_up(MGSweepT<T> a)
+template <typename T, int P, bool ZPER, bool FZ2, bool EXACT>
+__device__ __forceinline__ unsigned mg_up(const MGSweepT<T> &a, const MGCol<T, P, ZPER> &c)
 {
     extern __shared__ double mg_lds[];
-    MGCol<T, P, ZPER> c;
-    if (!c.init(a)) return;
+    unsigned least = ~0u;
     const int SL = a.rows * mg_lds_row<P>(a.pairs);
     // half planes: corrected black, first red and black, second red
     T *const L1 = reinterpret_cast<T *>(mg_lds), *const L2 = L1 + 2 * SL, *const L3 = L2 + 2 * SL,
@@ -495,7 +524,7 @@ __global__ void __launch_bounds__(kMGSweepThreads) k_mg_up(MGSweepT<T> a)
         c.template sum<PAR>(a, L1 + o * SL, xw[e], x0, wm, s);
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            r1[q] = c.template quot<PAR>(dg[m1], q, fr[m1][q] + s[q], d);
+            r1[q] = c.template quot<PAR, EXACT>(dg[m1], q, fr[m1][q] + s[q], d, least);
             x1[q] = a.cx * r1[q];
             xw[e][q] = x0[q];
             wm[q] = w[q];
@@ -506,7 +535,7 @@ __global__ void __launch_bounds__(kMGSweepThreads) k_mg_up(MGSweepT<T> a)
         c.template sum<PAR>(a, L2 + e * SL, xr1[o], x1, r1m, s);
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            b1[q] = c.template quot<PAR>(dg[m2], q, fb[m2][q] + s[q], d);
+            b1[q] = c.template quot<PAR, EXACT>(dg[m2], q, fb[m2][q] + s[q], d, least);
             x2[q] = a.cx * b1[q];
             xr1[o][q] = x1[q];
             r1m[q] = r1[q];
@@ -517,7 +546,7 @@ __global__ void __launch_bounds__(kMGSweepThreads) k_mg_up(MGSweepT<T> a)
         c.template sum<PAR>(a, L3 + o * SL, xb1[e], x2, b1m, s);
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            r2[q] = c.template quot<PAR>(dg[m3], q, fr[m3][q] + s[q], d);
+            r2[q] = c.template quot<PAR, EXACT>(dg[m3], q, fr[m3][q] + s[q], d, least);
             x3[q] = a.cx * r2[q];
             xb1[e][q] = x2[q];
             b1m[q] = b1[q];
@@ -530,7 +559,7 @@ __global__ void __launch_bounds__(kMGSweepThreads) k_mg_up(MGSweepT<T> a)
             c.template sum<PAR>(a, L4 + e * SL, xr2[o], x3, r2m, s);
 #pragma unroll
             for (int q = 0; q < P; ++q) {
-                out[2 * q + PAR] = c.template quot<PAR>(d4, q, f4[q] + s[q], d);
+                out[2 * q + PAR] = c.template quot<PAR, EXACT>(d4, q, f4[q] + s[q], d, least);
                 out[2 * q + 1 - PAR] = r2m[q];
             }
             mg_put(a.u + (size_t)i4 * fplane + (c.j * a.nz + 2 * c.kk0), out);
@@ -555,9 +584,19 @@ __global__ void __launch_bounds__(kMGSweepThreads) k_mg_up(MGSweepT<T> a)
             if (++t >= steps) break;
         }
     };
-    // as in k_mg_down; plane i's black cells have the other parity
+    // as in mg_down; plane i's black cells have the other parity
     if (__builtin_amdgcn_readfirstlane(c.par0)) march(MGInt<0>());
     else march(MGInt<1>());
+    return least;
+}
+template <typename T, int P, bool ZPER, bool FZ2>
+__global__ void __launch_bounds__(kMGSweepThreads) k_mg_up(MGSweepT<T> a)
+{
+    MGCol<T, P, ZPER> c;
+    if (!c.init(a)) return;
+    mg_exactly(a, [&](auto exact) {
+        return mg_up<T, P, ZPER, FZ2, decltype(exact)::value>(a, c);
+    });
 }
 
 } // namespace cfdmx
