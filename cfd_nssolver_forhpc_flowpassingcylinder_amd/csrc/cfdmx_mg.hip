@@ -636,11 +636,21 @@ static void launch_sweep(hipStream_t s, const MGSweepT<T> &a, bool down)
     }
 }
 
+// Whether a thread may take P z-pairs of a level.  In double with walls two spill up to 157
+// registers: a step of 384x192x96 cells took 5.58 ms, 4.85 with one and 5.03 with separate half
+// sweeps, one of 128x128x128 7.24, 5.53 and 6.58.  With periodic z two spill at most 32
+// (coarsening in all directions) and are up to 10% slower or 7% faster than one by the grid;
+// float's four with walls spill 29 and are level with two or up to 9% faster.
+template <typename T> constexpr bool mg_pairs(int P, bool zper)
+{
+    return std::is_same<T, float>::value || P == 1 || (P == 2 && zper);
+}
+
 // The tiling of a level for the one-pass kernels, from an estimate of a block's step: a CU
 // with W waves resident takes lat + add W us for a plane, or W issue us where the
 // instructions bound it (fitted to both kernels over 15 level shapes from 96x48x6 to
 // 1024x512x128, every P, ty and cxl: the choice is within 0.3% of the best measured one in
-// the mean).  More rows and planes a block mean fewer formed twice; more blocks fill the CUs.
+// the mean of these).  More rows and planes a block mean fewer formed twice; more blocks fill the CUs.
 struct SweepCost {
     double lat, add, issue;
     int waves; // of this kernel a CU holds (registers)
@@ -733,8 +743,8 @@ void mg_plan(MGLevelT<T> *L, int nlev)
         const MGSweepT<T> a = sweep_args(L[l], L[l + 1]);
         double best = 1e30;
         sweep_try<T, 1>(a, best, L[l]);
-        sweep_try<T, 2>(a, best, L[l]);
-        if (std::is_same<T, float>::value) sweep_try<T, 4>(a, best, L[l]);
+        if (mg_pairs<T>(2, L[l].zper)) sweep_try<T, 2>(a, best, L[l]);
+        if (mg_pairs<T>(4, L[l].zper)) sweep_try<T, 4>(a, best, L[l]);
     }
 }
 
@@ -744,11 +754,13 @@ static void launch_half_cycle(hipStream_t s, const MGLevelT<T> &F, const MGSweep
 {
     auto go = [&](auto zper) {
         constexpr bool Z = decltype(zper)::value;
-        if constexpr (std::is_same<T, float>::value) {
+        if constexpr (mg_pairs<T>(4, Z)) {
             if (P == 4) return launch_sweep<T, 4, Z>(s, a, down);
         }
-        if (P == 2) launch_sweep<T, 2, Z>(s, a, down);
-        else launch_sweep<T, 1, Z>(s, a, down);
+        if constexpr (mg_pairs<T>(2, Z)) {
+            if (P == 2) return launch_sweep<T, 2, Z>(s, a, down);
+        }
+        launch_sweep<T, 1, Z>(s, a, down);
     };
     if (F.zper) go(std::true_type());
     else go(std::false_type());
