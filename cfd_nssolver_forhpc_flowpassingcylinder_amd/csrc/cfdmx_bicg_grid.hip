@@ -29,11 +29,17 @@
 // (PRE = 1: 62 -> 31).  What is left is the three waits, about 2 us each, and the arithmetic
 // of a block's cells on one CU.
 //
-// All blocks have to be resident at once: the launch is cooperative, which fails where they
-// cannot be, and the caller keeps two such launches of one process apart.  Every wait is
-// bounded all the same (kMaxPolls, seconds): a block that gives up raises `failed` and
-// returns, as then do all others, and the caller solves again by launched phases.
+// All blocks have to be resident at once.  bicg_grid_cus takes no grid whose blocks the device
+// cannot hold, and the caller has no more resident kernels of a process on a device than leave
+// every block of each a CU of its own, so that a block that is not placed yet finds a CU without
+// one; other kernels end by themselves.  (A cooperative launch would ask for the same, but the
+// runtime has one queue for those: four contexts' 300 iterations at 64x40x8 take 17.6 ms so, 8.9
+// by ordinary launches.)  Every wait is bounded all the same (kMaxPolls, seconds): a block that
+// gives up raises `failed` and returns, as then do all others, and the caller solves again by
+// launched phases.
 #include "cfdmx_bicg.hpp"
+
+#include <algorithm>
 
 namespace cfdmx {
 
@@ -560,22 +566,25 @@ static size_t grid_lds(const Geo &g)
 
 int bicg_grid_slots(const Geo &g) { return 5 * g.nmarch * (1 + (grid_halves(g) ? kThreads : 0)); }
 
-bool bicg_grid_fits(const Geo &g, int pre, int uni)
+int bicg_grid_cus(const Geo &g, int pre, int uni, int &cus)
 {
     // one partial per polling thread, the rows beside the tile in kGridHalo cells a thread
     const int PL = grid_halves(g) ? kChunk / 2 : kChunk;
-    if (g.nmarch > kThreads || 2 * PL * g.nzc > kGridHalo * grid_threads(g)) return false;
-    int dev = 0, cus = 0, coop = 0, per = 0;
+    if (g.nmarch > kThreads || 2 * PL * g.nzc > kGridHalo * grid_threads(g)) return 0;
+    int dev = 0, per = 0;
     const void *k = grid_kernel(g, pre, uni);
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess ||
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, grid_threads(g), grid_lds(g)) !=
             hipSuccess) {
         (void)hipGetLastError();
-        return false;
+        return 0;
     }
-    return coop && per > 0 && (long long)per * cus >= grid_blocks_of(g);
+    const int blocks = grid_blocks_of(g);
+    if ((long long)per * cus < blocks) return 0;
+    // workgroups are dealt to the 8 XCDs in turn, so the blocks of one count as those of the
+    // fullest; more than one a CU leave no room beside them
+    return std::min((blocks + 7) / 8 * 8, cus);
 }
 
 hipError_t launch_bicg_grid(const Geo &g, hipStream_t s, int pre, int uni, BicgBuffers &B,
@@ -588,9 +597,8 @@ hipError_t launch_bicg_grid(const Geo &g, hipStream_t s, int pre, int uni, BicgB
     Geo geo = g;
     BicgBuffers buf = B;
     void *args[] = {&geo, &buf, &x, &partC, &slots, &st, &failed, &m0, &count};
-    const void *k = grid_kernel(g, pre, uni);
-    return hipLaunchCooperativeKernel(k, dim3(grid_blocks_of(g)), dim3(grid_threads(g)), args,
-                                      (unsigned)grid_lds(g), s);
+    return hipLaunchKernel(grid_kernel(g, pre, uni), dim3(grid_blocks_of(g)),
+                           dim3(grid_threads(g)), args, grid_lds(g), s);
 }
 
 } // namespace cfdmx

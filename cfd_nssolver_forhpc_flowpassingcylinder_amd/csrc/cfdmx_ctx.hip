@@ -6,6 +6,7 @@
 #include <atomic>
 #include <chrono>
 #include <cmath>
+#include <condition_variable>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
@@ -120,6 +121,7 @@ struct cfdmx_ctx {
     // resident BiCGSTAB (cfdmx_bicg_grid.hip): where the grid takes it, its partial sums'
     // slots and its failure flag
     int grid_solve = 0, grid_uni = 0;
+    int grid_cus = 0, device_cus = 0; // CUs a launch holds, and all there are
     unsigned long long *grid_slots = nullptr;
     KState *grid_keep = nullptr;
     int *grid_failed = nullptr, *grid_failed_h = nullptr;
@@ -176,8 +178,39 @@ static __device__ __align__(256) double scratch[2 * kScratchBlocks];
 constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
 static double *g_scratch[kMaxDevices] = {};
-// one resident BiCGSTAB kernel at a time on a device (solve_bicgstab_core)
-static std::mutex g_grid_mu[kMaxDevices];
+// The CUs of a device that resident BiCGSTAB kernels hold (solve_bicgstab_core).  Two that do
+// not fit side by side might each hold CUs that the other waits for, so a launch waits for its
+// own, in turn: first come, first served, or a large one might wait behind small ones for good.
+class GridRoom {
+    std::mutex mu;
+    std::condition_variable cv;
+    unsigned long long tickets = 0, turn = 0;
+    int held = 0;
+
+public:
+    void take(int n, int cus)
+    {
+        std::unique_lock<std::mutex> lock(mu);
+        const unsigned long long mine = tickets++;
+        cv.wait(lock, [&] { return turn == mine && (held == 0 || held + n <= cus); });
+        ++turn;
+        held += n;
+        cv.notify_all();
+    }
+    void give(int n)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        held -= n;
+        cv.notify_all();
+    }
+};
+static GridRoom g_grid_room[kMaxDevices];
+struct GridHold {
+    GridRoom &room;
+    const int n;
+    GridHold(GridRoom &r, int cus, int device_cus) : room(r), n(cus) { room.take(n, device_cus); }
+    ~GridHold() { room.give(n); }
+};
 
 #define FAIL(code, ...)                                                                        \
     do {                                                                                       \
@@ -736,8 +769,9 @@ static int setup_device(cfdmx_ctx *ctx)
         for (int q = 0; q < 2; ++q)
             for (int i = 0; i < nc[a]; ++i)
                 if (buf[poff[a][q] + i] != buf[poff[a][q]]) ctx->grid_uni = 0;
-    ctx->grid_solve =
-        c.precision == CFDMX_PRECISION_FP64 && bicg_grid_fits(g, c.precond, ctx->grid_uni) ? 1 : 0;
+    if (c.precision == CFDMX_PRECISION_FP64)
+        ctx->grid_cus = bicg_grid_cus(g, c.precond, ctx->grid_uni, ctx->device_cus);
+    ctx->grid_solve = ctx->grid_cus > 0;
     if (ctx->grid_solve) {
         ALLOC(ctx->grid_slots, (size_t)bicg_grid_slots(g));
         ALLOC(ctx->grid_keep, 1);
@@ -1436,9 +1470,9 @@ static int solve_bicgstab_core(cfdmx_ctx *ctx, const SolveTarget &T, int *iters,
         constexpr int kGridBatch = 1024;
         hipError_t e = hipSuccess;
         {
-            // two resident kernels of a device might each hold CUs that the other waits for
-            std::lock_guard<std::mutex> one(
-                g_grid_mu[ctx->device >= 0 && ctx->device < kMaxDevices ? ctx->device : 0]);
+            const GridHold hold(
+                g_grid_room[ctx->device >= 0 && ctx->device < kMaxDevices ? ctx->device : 0],
+                ctx->grid_cus, ctx->device_cus);
             PROF(CFDMX_K_BICG_A,
                  e = launch_bicg_grid(g, s, pre, ctx->grid_uni, ctx->B, T.x, ctx->bpart[2],
                                       ctx->grid_slots, T.kst, ctx->grid_keep, ctx->grid_failed, m,
