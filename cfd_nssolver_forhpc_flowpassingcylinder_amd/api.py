@@ -32,7 +32,8 @@ EXPORTS = [
     "cfdmx_bc_copy", "cfdmx_pressure_rhs", "cfdmx_solve_bicgstab", "cfdmx_solve_rbsor",
     "cfdmx_transform", "cfdmx_project_ib", "cfdmx_swap_t0_t3", "cfdmx_cd_cl", "cfdmx_cfl",
     "cfdmx_apply_operator", "cfdmx_apply_operator_transpose", "cfdmx_step",
-    "cfdmx_synchronize", "cfdmx_profile", "cfdmx_profile_read", "cfdmx_set_tolerance", "cfdmx_set_physics", "cfdmx_upload_force",
+    "cfdmx_synchronize", "cfdmx_profile", "cfdmx_profile_read", "cfdmx_resident_solve",
+    "cfdmx_set_tolerance", "cfdmx_set_physics", "cfdmx_upload_force",
     "cfdmx_drag_objective", "cfdmx_adjoint_drag", "cfdmx_plot3d_q", "cfdmx_plot3d_flush",
     "cfdmx_plot3d_x", "cfdmx_checkpoint_save", "cfdmx_checkpoint_load", "cfdmx_smagorinsky",
     "cfdmx_download_viseff", "cfdmx_cd_cl_noalloc",
@@ -131,6 +132,7 @@ def load_library(path=LIB_PATH):
     L.cfdmx_apply_operator_transpose.argtypes = [vp, DP, DP]
     L.cfdmx_step.argtypes = [vp, C.c_int, C.POINTER(StepInfo)]
     L.cfdmx_profile.argtypes = [vp, C.c_int]
+    L.cfdmx_resident_solve.argtypes = [vp, C.c_int, C.POINTER(C.c_int)]
     L.cfdmx_set_tolerance.argtypes = [vp, C.c_double, C.c_int]
     L.cfdmx_set_physics.argtypes = [vp, C.c_double, C.c_double]
     L.cfdmx_profile_read.argtypes = [vp, C.c_int, DP, C.POINTER(C.c_longlong)]
@@ -403,6 +405,13 @@ class FlowSolver:
 
     def profile(self, enable):
         self._chk(self.L.cfdmx_profile(self.h, 1 if enable else 0), "profile")
+
+    def resident_solve(self, launches=-1):
+        """Solves so far that left the resident kernel for launched phases; launches >= 0:
+        later launches of a solve give up at once (for tests)."""
+        n = C.c_int()
+        self._chk(self.L.cfdmx_resident_solve(self.h, launches, C.byref(n)), "resident_solve")
+        return n.value
 
     def profile_read(self):
         """{kernel: (total_ms, launches)} for every kernel class"""

@@ -46,7 +46,6 @@ namespace cfdmx {
 // a quiet NaN that no arithmetic produces (its payload is set); a partial that is this very
 // value is written as the plain NaN
 constexpr unsigned long long kEmpty = 0x7ff8dead5eed0001ull;
-constexpr int kMaxPolls = 1 << 21;
 constexpr int kGridHalo = 2; // cells of the rows beside the tile that one thread holds
 
 __device__ __forceinline__ void put_through(double *p, double v)
@@ -81,7 +80,7 @@ __global__ void k_grid_slots(int n, unsigned long long *slots, const KState *st,
 template <int PRE, int T, int NC, int PL, bool UNI>
 __global__ void __launch_bounds__(T)
 k_bicg_grid(Geo g, BicgBuffers B, double *__restrict__ x, double *partC,
-            unsigned long long *slots, KState *st, int *failed, int m0, int count)
+            unsigned long long *slots, KState *st, int *failed, int polls, int m0, int count)
 {
     static_assert(PL == kChunk || 2 * PL == kChunk, "whole or half march blocks");
     extern __shared__ double lds[];
@@ -264,7 +263,7 @@ k_bicg_grid(Geo g, BicgBuffers B, double *__restrict__ x, double *partC,
             double acc = 0.0;
             if (second) {
                 unsigned long long v = kEmpty;
-                for (int q = 0; q < kMaxPolls && v == kEmpty; ++q)
+                for (int q = 0; q < polls && v == kEmpty; ++q)
                     v = __hip_atomic_load(chain + k * kThreads + w, __ATOMIC_RELAXED,
                                           __HIP_MEMORY_SCOPE_AGENT);
                 if (v == kEmpty) gave_up = 1;
@@ -297,7 +296,8 @@ k_bicg_grid(Geo g, BicgBuffers B, double *__restrict__ x, double *partC,
         if (tid < kThreads) {
             unsigned long long v[2] = {0, 0};
             if (tid < nb) {
-                for (int w = 0; w < kMaxPolls; ++w) {
+                v[0] = kEmpty;
+                for (int w = 0; w < polls; ++w) {
                     v[0] = __hip_atomic_load(slot + ns * tid, __ATOMIC_RELAXED,
                                              __HIP_MEMORY_SCOPE_AGENT);
                     if (ns == 2)
@@ -589,14 +589,14 @@ int bicg_grid_cus(const Geo &g, int pre, int uni, int &cus)
 
 hipError_t launch_bicg_grid(const Geo &g, hipStream_t s, int pre, int uni, BicgBuffers &B,
                             double *x, double *partC, unsigned long long *slots, KState *st,
-                            KState *keep, int *failed, int m0, int count)
+                            KState *keep, int *failed, int polls, int m0, int count)
 {
     const int n = bicg_grid_slots(g);
     hipLaunchKernelGGL(k_grid_slots, dim3((n + 255) / 256), dim3(256), 0, s, n, slots,
                        (const KState *)st, m0 == 0 ? keep : nullptr);
     Geo geo = g;
     BicgBuffers buf = B;
-    void *args[] = {&geo, &buf, &x, &partC, &slots, &st, &failed, &m0, &count};
+    void *args[] = {&geo, &buf, &x, &partC, &slots, &st, &failed, &polls, &m0, &count};
     return hipLaunchKernel(grid_kernel(g, pre, uni), dim3(grid_blocks_of(g)),
                            dim3(grid_threads(g)), args, grid_lds(g), s);
 }

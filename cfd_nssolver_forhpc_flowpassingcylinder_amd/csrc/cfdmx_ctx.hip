@@ -125,6 +125,9 @@ struct cfdmx_ctx {
     unsigned long long *grid_slots = nullptr;
     KState *grid_keep = nullptr;
     int *grid_failed = nullptr, *grid_failed_h = nullptr;
+    // launches of a solve after which the others give up (< 0: none do), solves that launched
+    // phases began again
+    int grid_give_up = -1, grid_fallbacks = 0;
     double *scal = nullptr; // [0] cfl, [1] cd, [2] cl, [3..5] max(T0 - T3) of u, v, w
     double *inflow = nullptr;
     KState *kst = nullptr;
@@ -1453,6 +1456,10 @@ struct SolveTarget {
     KState *kst, *kst_h;
 };
 
+// looks at a partial sum before a block of the resident kernel gives up (about a microsecond
+// each, of waits that take two or three)
+constexpr int kGridPolls = 1 << 21;
+
 static int solve_bicgstab_core(cfdmx_ctx *ctx, const SolveTarget &T, int *iters, double *res)
 {
     hipStream_t s = ctx->stream;
@@ -1468,6 +1475,7 @@ static int solve_bicgstab_core(cfdmx_ctx *ctx, const SolveTarget &T, int *iters,
     // last (11 to 31 us each); a solve that ends earlier ends the kernel
     while (ctx->grid_solve) {
         constexpr int kGridBatch = 1024;
+        const bool give_up = ctx->grid_give_up >= 0 && m >= ctx->grid_give_up * kGridBatch;
         hipError_t e = hipSuccess;
         {
             const GridHold hold(
@@ -1475,8 +1483,8 @@ static int solve_bicgstab_core(cfdmx_ctx *ctx, const SolveTarget &T, int *iters,
                 ctx->grid_cus, ctx->device_cus);
             PROF(CFDMX_K_BICG_A,
                  e = launch_bicg_grid(g, s, pre, ctx->grid_uni, ctx->B, T.x, ctx->bpart[2],
-                                      ctx->grid_slots, T.kst, ctx->grid_keep, ctx->grid_failed, m,
-                                      kGridBatch));
+                                      ctx->grid_slots, T.kst, ctx->grid_keep, ctx->grid_failed,
+                                      give_up ? 0 : kGridPolls, m, kGridBatch));
             if (e == hipSuccess) {
                 HIPCHK(hipMemcpyAsync(T.kst_h, T.kst, sizeof(KState), hipMemcpyDeviceToHost, s));
                 HIPCHK(hipMemcpyAsync(ctx->grid_failed_h, ctx->grid_failed, sizeof(int),
@@ -1490,6 +1498,7 @@ static int solve_bicgstab_core(cfdmx_ctx *ctx, const SolveTarget &T, int *iters,
             // solve again from its start, this context's solves by launched phases from here
             (void)hipGetLastError();
             ctx->grid_solve = 0;
+            ++ctx->grid_fallbacks;
             *ctx->grid_failed_h = 0;
             launch_set_int(s, ctx->grid_failed, 0);
             launch_copy(s, g.N, *T.px1, T.x);
@@ -1991,6 +2000,14 @@ int cfdmx_synchronize(cfdmx_ctx *ctx)
     if (!ctx) return CFDMX_ERR_ARG;
     HIPCHK(hipStreamSynchronize(ctx->stream));
     prof_harvest(ctx);
+    return CFDMX_OK;
+}
+
+int cfdmx_resident_solve(cfdmx_ctx *ctx, int launches, int *fallbacks)
+{
+    if (!ctx) return CFDMX_ERR_ARG;
+    ctx->grid_give_up = launches < 0 ? -1 : std::min(launches, 1 << 20);
+    if (fallbacks) *fallbacks = ctx->grid_fallbacks;
     return CFDMX_OK;
 }
 

@@ -325,6 +325,13 @@ CFDMX_API int cfdmx_adjoint_drag(cfdmx_ctx *ctx, int nsteps, int checkpoint_ever
 /* Enable (1) or disable (0) HIP-event timing of every launch of the kernels above on
  * the context's stream; resets the totals. */
 CFDMX_API int cfdmx_profile(cfdmx_ctx *ctx, int enable);
+/* FP64 BiCGSTAB on small grids runs in one resident kernel for up to 1024 iterations a
+ * launch, whose workgroups wait for each other.  A solve whose workgroups wait in vain for
+ * seconds (others hold the device) is done again from its start by launched phases, with the
+ * same bits, and so are the context's later solves.  *fallbacks (may be NULL): how often that
+ * has happened.  launches >= 0: the launches of a solve after that many give up at once,
+ * which takes the solve there (for tests); negative, as created: none does. */
+CFDMX_API int cfdmx_resident_solve(cfdmx_ctx *ctx, int launches, int *fallbacks);
 /* Accumulated device time and launch count of one kernel class. */
 CFDMX_API int cfdmx_profile_read(cfdmx_ctx *ctx, int kernel, double *total_ms, long long *launches);
 
