@@ -1,6 +1,7 @@
 // cfdmx_bicg_grid.hip -- the BiCGSTAB iteration of small grids as one resident kernel
-// (bicgstabRe2.hpp:82-180): at most 128 march blocks of tiles over 512 cells (a million
-// cells), or 256 of smaller ones.
+// (bicgstabRe2.hpp:82-180): grids whose workgroups the device holds all at once.  On 256 CUs
+// that is up to 128 march blocks of tiles over 512 cells (a million cells, two workgroups each),
+// or 256 of smaller ones.
 //
 // Launched phase by phase, such a grid's iteration is bound by latency: a march block takes
 // its 8 planes one after the other (phases A, B, C 13, 12 and 6 us at 128x64x4, 19, 17 and
@@ -70,9 +71,9 @@ __global__ void k_grid_slots(int n, unsigned long long *slots, const KState *st,
 }
 
 // T threads a block, NC columns of the plane tile each (T * NC is at least the tile's cells).
-// UNI: every block holds 8 planes and a whole tile, and every row has the same coefficients (a
-// uniform grid), so that they are scalars and a row's diagonal is one of three values per
-// column.
+// UNI (bicg_grid_uni): every block holds 8 planes and a whole tile, and every row has the same
+// coefficients (a uniform grid), so that they are scalars and a row's diagonal is one of three
+// values per column.
 //
 // A column or plane that does not exist holds zeros throughout: its coefficients towards the
 // others are zeros, so that it takes part in the arithmetic without a branch, and only the
@@ -565,6 +566,19 @@ static size_t grid_lds(const Geo &g)
 }
 
 int bicg_grid_slots(const Geo &g) { return 5 * g.nmarch * (1 + (grid_halves(g) ? kThreads : 0)); }
+
+// UNI: every row has the same coefficients (element 0 of each axis's), every march block holds
+// 8 planes, and every thread's column exists
+int bicg_grid_uni(const Geo &g, const double *const (&coef)[3][2])
+{
+    const int n[3] = {g.nxc, g.nyc, g.nzc};
+    for (int a = 0; a < 3; ++a)
+        for (int q = 0; q < 2; ++q)
+            for (int i = 0; i < n[a]; ++i)
+                if (coef[a][q][i] != coef[a][q][0]) return 0;
+    return g.nxc % kChunk == 0 &&
+           (g.cyz % kTile == 0 || g.cyz == kThreads || g.cyz == 2 * kThreads);
+}
 
 int bicg_grid_cus(const Geo &g, int pre, int uni, int &cus)
 {

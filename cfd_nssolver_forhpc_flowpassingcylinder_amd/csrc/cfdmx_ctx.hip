@@ -766,12 +766,12 @@ static int setup_device(cfdmx_ctx *ctx)
         HIPCHK(hipMemset(ctx->viseff, 0, N * sizeof(double)));
     }
     for (int q = 0; q < 3; ++q) ALLOC(ctx->bpart[q], 2 * (size_t)g.nmarch + 64);
-    // one set of coefficients for every row, whole tiles and whole blocks of planes
-    ctx->grid_uni = c.nx % kChunk == 0 && (g.cyz % kTile == 0 || g.cyz == 256 || g.cyz == 512);
-    for (int a = 0; a < 3; ++a)
-        for (int q = 0; q < 2; ++q)
-            for (int i = 0; i < nc[a]; ++i)
-                if (buf[poff[a][q] + i] != buf[poff[a][q]]) ctx->grid_uni = 0;
+    {
+        const double *coef[3][2];
+        for (int a = 0; a < 3; ++a)
+            for (int q = 0; q < 2; ++q) coef[a][q] = &buf[poff[a][q]];
+        ctx->grid_uni = bicg_grid_uni(g, coef);
+    }
     if (c.precision == CFDMX_PRECISION_FP64)
         ctx->grid_cus = bicg_grid_cus(g, c.precond, ctx->grid_uni, ctx->device_cus);
     ctx->grid_solve = ctx->grid_cus > 0;

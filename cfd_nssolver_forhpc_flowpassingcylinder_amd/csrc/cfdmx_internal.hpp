@@ -95,13 +95,16 @@ template <typename T>
 void launch_bicg_C(const Geo &g, hipStream_t s, BicgBuf<T> &B, T *x, double *const part[3],
                    KState *st, int m);
 void launch_bicg_check(const Geo &g, hipStream_t s, double *const part[3], KState *st, int m);
-// iterations m0 .. m0 + count - 1 in one resident kernel (cfdmx_bicg_grid.hip), on grids for
-// which bicg_grid_cus is not 0 (uni: every row has the same x coefficients); partC: 2 * nmarch doubles kept from launch to launch of a solve,
-// slots: bicg_grid_slots values, keep: takes the state the solve starts with (m0 = 0),
-// failed: set to 1 by a block that waited in vain, having looked `polls` times
 // CUs a launch has to itself among resident kernels of a device; cus: of the device
 int bicg_grid_cus(const Geo &g, int pre, int uni, int &cus);
+// coef: host copies of PAxis m and p of each axis
+int bicg_grid_uni(const Geo &g, const double *const (&coef)[3][2]);
 int bicg_grid_slots(const Geo &g);
+// iterations m0 .. m0 + count - 1 in one resident kernel (cfdmx_bicg_grid.hip), on grids for
+// which bicg_grid_cus is not 0.  uni: what bicg_grid_uni says of the grid; partC: 2 * nmarch
+// doubles kept from launch to launch of a solve, slots: bicg_grid_slots values, keep: takes the
+// state the solve starts with (m0 = 0), failed: set to 1 by a block that waited in vain, having
+// looked `polls` times
 hipError_t launch_bicg_grid(const Geo &g, hipStream_t s, int pre, int uni, BicgBuffers &B,
                             double *x, double *partC, unsigned long long *slots, KState *st,
                             KState *keep, int *failed, int polls, int m0, int count);
