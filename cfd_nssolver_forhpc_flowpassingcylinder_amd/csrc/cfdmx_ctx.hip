@@ -136,6 +136,8 @@ struct cfdmx_ctx {
     // red-black SOR working set of a context configured for it (even nzc): p of both
     // colours, then the right-hand side of both colours, in one allocation
     double *sorw = nullptr;
+    // passes of two sweeps: p's other copy (sorw then holds the right-hand side and the maxima)
+    double *sor_other = nullptr;
     SorState *sorst = nullptr;
     SorPlan sorp = {}; // passes of two sweeps, in contexts configured for red-black SOR
     int *count = nullptr;
@@ -738,7 +740,8 @@ static int setup_device(cfdmx_ctx *ctx)
         HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
         ctx->sorp = sor_plan(g, ctx->sorc, cus);
         if (ctx->sorp.blocks) {
-            ALLOC(ctx->sorw, G + G % 2 + N + 4 * (size_t)ctx->sorp.blocks);
+            ALLOC(ctx->sor_other, G);
+            ALLOC(ctx->sorw, N + 4 * (size_t)ctx->sorp.blocks);
             ALLOC(ctx->sorst, 2);
         } else if (g.nzc % 2 == 0) {
             ALLOC(ctx->sorw, 2 * N);
@@ -1714,8 +1717,8 @@ static int solve_rbsor_passes(cfdmx_ctx *ctx)
     hipStream_t s = ctx->stream;
     const Geo &g = ctx->g;
     const SorPlan &pl = ctx->sorp;
-    double *buf[2] = {ctx->p, ctx->sorw};
-    double *rhs = ctx->sorw + g.G + g.G % 2;
+    double *buf[2] = {ctx->p, ctx->sor_other};
+    double *rhs = ctx->sorw;
     double *part[2] = {rhs + g.N, rhs + g.N + 2 * (size_t)pl.blocks};
     const auto pass = [&](int from, const SorTurn &turn) {
         PROF(CFDMX_K_SOR, launch_sor_pass(g, s, pl, ctx->cfg.sor_omega, ctx->sorc, rhs,
@@ -1741,7 +1744,7 @@ static int solve_rbsor_passes(cfdmx_ctx *ctx)
     // that sweep alone is run again from there
     const int from = ((ctx->sst_h->iters - 1) / 2) & 1;
     if (ctx->sst_h->iters & 1) pass(from, {nullptr, nullptr, nullptr, part[0], 1});
-    if (from == 0) launch_copy(s, g.G, buf[1], buf[0]);
+    if (from == 0) std::swap(ctx->p, ctx->sor_other);
     LAUNCHCHK();
     return CFDMX_OK;
 }
