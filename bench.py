@@ -45,8 +45,11 @@ BYTES_PER_CELL = {
     "convdiff": 48,  # r u, v, w;  w u*, v*, w*
     "rhs": 32,       # r u*, v*, w*;  w b
     "project": 96,   # r u*, v*, w*, X, eta;  w u, v, w, p, f(3)
-    "sor_half": 24,  # pass of two red-black sweeps: r p, rhs;  w p
+    "sor_half": 16,  # half sweep: r the other colour, own p, rhs;  w own p
 }
+SOR_PASS_BYTES = 24  # two red-black sweeps in one launch: r p, rhs;  w p
+# an iteration of the resident solve: r x;  w x (the other vectors stay on the CUs)
+RESIDENT_BYTES = 16
 
 # the BiCGSTAB iteration (phases A + B + C) is the FP64 step's dominant work: 128 B/cell
 # per iteration (32 + 24 + 72)
@@ -320,13 +323,15 @@ def run_mode(wl, args, precision):
     # per-kernel device time from HIP events on the library's stream, over further
     # steps of the same run (events are kept out of the wall-clock region)
     s.profile(True)
+    done = 0  # iterations (sweeps) the profiled steps ran
     for q in range(args.profile_steps):
-        s.step(1)
+        info = s.step(1)
+        done += (info["iters"] + 1) * info["solved"]
         print(f"{tag} profiled step {q + 1}", file=sys.stderr, flush=True)
     s.synchronize()
     prof = s.profile_read()
     s.profile(False)
-    return s, warm, infos, wall, prof
+    return s, warm, infos, wall, prof, done
 
 
 # gradients of the time-averaged drag: 256 x 128 x 32, Re 100, 50 steps, checkpoints
@@ -617,37 +622,42 @@ def rbsor_run(wl, args):
     s.synchronize()
     wall = time.perf_counter() - t
     s.profile(True)
-    s.step(1)
+    done = s.step(1)["iters"] + 1
     s.synchronize()
     prof = s.profile_read()
     s.profile(False)
     s.close()
     n_cells = wl["nx"] * wl["ny"] * wl["nz"]
+    table = launch_bytes(prof, done)
+    passes = table["sor_half"] == SOR_PASS_BYTES
     ms, launches = prof["sor_half"]
     avg_s = ms / 1e3 / launches
-    achieved = BYTES_PER_CELL["sor_half"] * n_cells / avg_s / 1e9
+    achieved = table["sor_half"] * n_cells / avg_s / 1e9
     sweeps = [i["iters"] + 1 for i in infos]
     return {
         "value": round(n_cells * args.steps / wall / 1e6, 4), "unit": "Mcell-steps/s",
         "ms_per_step": round(wall / args.steps * 1e3, 3),
         "config": (f"{wl['nx']}x{wl['ny']}x{wl['nz']}, Re={wl['re']:g}, dt={wl['dt']:g}, "
                    f"red-black SOR omega 1.8, tol {wl['tol']:g} (max |dp| per sweep), at most "
-                   f"{args.sor_maxit} sweeps per step, FP64, two sweeps a pass"),
+                   f"{args.sor_maxit} sweeps per step, FP64"
+                   + (", two sweeps a pass" if passes else "")),
         "sweep_cap": args.sor_maxit,
         "sweeps_per_step": sweeps, "max_dp_per_step": [i["err"] for i in infos],
         "steps_reaching_tol": sum(1 for i in infos if i["err"] < wl["tol"]),
         "ms_per_sweep": round(wall / sum(sweeps) * 1e3, 4),
-        "roofline": {"bound": "hbm", "kernel": "k_sor_pass (two sweeps)",
+        "roofline": {"bound": "hbm",
+                     "kernel": "k_sor_pass (two sweeps)" if passes else "k_sor_rb2 (half sweep)",
                      "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": measured_traffic(args.workload, "sor_pass"),
+                     "traffic": measured_traffic(args.workload,
+                                                 "sor_pass" if passes else "sor_half"),
                      "avg_launch_us": round(avg_s * 1e6, 2),
-                     "bytes_per_launch": BYTES_PER_CELL["sor_half"] * n_cells,
-                     "bytes_note": ("24 B per cell of the grid per pass: p and the "
-                                    "right-hand side read, p written (12 B/cell per full "
-                                    "sweep); what blocks read twice around their tiles is "
-                                    "not counted")},
-        "kernels": kernel_table(prof, n_cells, BYTES_PER_CELL),
+                     "bytes_per_launch": table["sor_half"] * n_cells,
+                     "bytes_note": ("pass: 24 B per cell of the grid, p and the right-hand side "
+                                    "read, p written (12 B/cell per full sweep); what blocks "
+                                    "read twice around their tiles is not counted.  Half "
+                                    "sweep: 16 B per cell of the grid")},
+        "kernels": kernel_table(prof, n_cells, table),
     }
 
 
@@ -829,6 +839,57 @@ def les_run(wl, args):
     return out
 
 
+def resident(prof):
+    """Whether one resident kernel ran the FP64 BiCGSTAB solves of a profile."""
+    return prof["bicg_A"][1] > 0 and prof["bicg_B"][1] == 0
+
+
+def launch_bytes(prof, done):
+    """BYTES_PER_CELL as the launches of a profile of `done` iterations (sweeps) were: red-black
+    SOR in passes of two sweeps takes fewer launches than sweeps and a batch, in half sweeps two
+    a sweep; a launch of the resident solve has no count of its own."""
+    table = dict(BYTES_PER_CELL)
+    if prof["sor_half"][1] < 2 * done:
+        table["sor_half"] = SOR_PASS_BYTES
+    if resident(prof):
+        del table["bicg_A"]
+    return table
+
+
+def step_roofline(prof, n_cells, workload, done):
+    """The dominant work by device time during the profiled steps, which ran `done` pressure
+    iterations: with BiCGSTAB the iteration, its three phase kernels together (128 B/cell), or
+    on small grids an iteration of the resident solve; otherwise the kernel class with the most
+    device time."""
+    table = launch_bytes(prof, done)
+    cands = {k: v for k, v in prof.items() if k in table and v[1] > 0}
+    bound = "hbm"
+    if all(k in cands for k in ITERATION_PHASES):
+        iters_run = min(cands[k][1] for k in ITERATION_PHASES)
+        avg_s = sum(cands[k][0] for k in ITERATION_PHASES) / 1e3 / iters_run
+        alg_bytes = sum(BYTES_PER_CELL[k] for k in ITERATION_PHASES) * n_cells
+        dom = "bicgstab_iteration (k_march<0> + k_march<1> + k_march_C)"
+        traffic = [measured_traffic(workload, k) for k in ITERATION_PHASES]
+        traffic = sum(traffic) if all(t is not None for t in traffic) else None
+    elif resident(prof) and done:
+        # exchanges between workgroups bound it, not memory
+        bound = "latency"
+        avg_s = prof["bicg_A"][0] / 1e3 / done
+        alg_bytes = RESIDENT_BYTES * n_cells
+        dom, traffic = "bicgstab_iteration (in k_bicg_grid)", None
+    else:
+        k0 = max(cands, key=lambda k: cands[k][0])
+        avg_s = cands[k0][0] / 1e3 / cands[k0][1]
+        alg_bytes = table[k0] * n_cells
+        name = "sor_pass" if k0 == "sor_half" and table[k0] == SOR_PASS_BYTES else k0
+        dom, traffic = name, measured_traffic(workload, name)
+    achieved = alg_bytes / avg_s / 1e9
+    return {"bound": bound, "kernel": dom, "achieved": round(achieved, 1),
+            "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
+            "traffic": traffic, "avg_launch_us": round(avg_s * 1e6, 2),
+            "bytes_per_launch": alg_bytes}
+
+
 def kernel_table(prof, n_cells, bytes_per_cell):
     return {k: {"ms_total": round(v[0], 3), "launches": v[1],
                 "avg_us": round(v[0] * 1e3 / v[1], 2) if v[1] else None,
@@ -924,7 +985,7 @@ def main():
                                              not args.no_fd)}), flush=True)
         return
     if args.part in ("mixed", "fp64mg"):
-        sm, mwarm, minfos, mwall, mprof = run_mode(wl, args, 1 if args.part == "mixed" else 2)
+        sm, mwarm, minfos, mwall, mprof, _ = run_mode(wl, args, 1 if args.part == "mixed" else 2)
         print(json.dumps({args.part: {
             "value": round(n_cells * args.steps / mwall / 1e6, 4), "unit": "Mcell-steps/s",
             "iters_per_step": [i["iters"] for i in minfos],
@@ -932,34 +993,13 @@ def main():
             "kernels": kernel_table(mprof, n_cells, BYTES_PER_CELL_FP32)}}), flush=True)
         sm.close()
         return
-    s, warm, infos, wall, prof = run_mode(wl, args, 0)
+    s, warm, infos, wall, prof, done = run_mode(wl, args, 0)
     value = n_cells * args.steps / wall / 1e6
     iters = [i["iters"] for i in infos]
     mean_iters = sum(iters) / max(1, len(iters))
 
-    # the dominant work by device time during the profiled steps: with BiCGSTAB the
-    # iteration, its three phase kernels together (128 B/cell per iteration); otherwise
-    # the kernel class with the most device time
-    cands = {k: v for k, v in prof.items() if k in BYTES_PER_CELL and v[1] > 0}
-    if all(k in cands for k in ITERATION_PHASES):
-        iters_run = min(cands[k][1] for k in ITERATION_PHASES)
-        avg_s = sum(cands[k][0] for k in ITERATION_PHASES) / 1e3 / iters_run
-        alg_bytes = sum(BYTES_PER_CELL[k] for k in ITERATION_PHASES) * n_cells
-        dom = "bicgstab_iteration (k_march<0> + k_march<1> + k_march_C)"
-        traffic = [measured_traffic(args.workload, k) for k in ITERATION_PHASES]
-        traffic = sum(traffic) if all(t is not None for t in traffic) else None
-    else:
-        k0 = max(cands, key=lambda k: cands[k][0])
-        avg_s = cands[k0][0] / 1e3 / cands[k0][1]
-        alg_bytes = BYTES_PER_CELL[k0] * n_cells
-        dom, traffic = k0, measured_traffic(args.workload, k0)
-    achieved = alg_bytes / avg_s / 1e9
-    roofline = {"bound": "hbm", "kernel": dom, "achieved": round(achieved, 1),
-                "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                "traffic": traffic,
-                "avg_launch_us": round(avg_s * 1e6, 2),
-                "bytes_per_launch": alg_bytes}
-    kernels = kernel_table(prof, n_cells, BYTES_PER_CELL)
+    roofline = step_roofline(prof, n_cells, args.workload, done)
+    kernels = kernel_table(prof, n_cells, launch_bytes(prof, done))
     ceiling = None if args.no_stream_ceiling else stream_ceiling_child(n_cells)
 
     mixed = None
@@ -988,11 +1028,11 @@ def main():
         # the same algorithm with the inner solve in FP64 (multigrid-preconditioned
         # BiCGSTAB, FP64 refinement): the converged FP64 solution and the precision-only
         # comparison
-        sg, gwarm, ginfos, gwall, gprof = run_mode(wl, args, 2)
+        sg, gwarm, ginfos, gwall, gprof, _ = run_mode(wl, args, 2)
         gvalue = n_cells * args.steps / gwall / 1e6
         refmg = fields(sg)
         sg.close()
-        sm, mwarm, minfos, mwall, mprof = run_mode(wl, args, 1)
+        sm, mwarm, minfos, mwall, mprof, _ = run_mode(wl, args, 1)
         mvalue = n_cells * args.steps / mwall / 1e6
         got = fields(sm)
         sm.close()
