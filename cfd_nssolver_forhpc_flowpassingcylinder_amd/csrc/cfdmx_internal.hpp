@@ -139,7 +139,9 @@ constexpr int kMGCoarseAxis = 512; // largest axis length of that level
 // (k_mg_tail).  A level with even nz in two one-pass launches takes 14 us at 64x32x2, level
 // with the workgroup's 13 us in float and ahead of its 20 us in double (V-cycles 173 against
 // 177 us and 238 against 252 us at 512x256x64); one with odd nz would take a launch per half
-// sweep, where the workgroup wins up to twice the size (55 against 70 us at 96x48x6)
+// sweep, where the workgroup wins up to twice the size, the most that its LDS holds (steps of
+// twelve grids with an odd level of 1024 to 4096 cells, 40x16x5 to 96x56x6: 1.3 to 1.4 times
+// as fast)
 constexpr int kMGTailCells = 2048, kMGTailCellsOdd = 4096;
 constexpr int kMGTailLevels = 8;
 

@@ -495,8 +495,8 @@ __global__ void k_pb_update_p(Geo g, int first, const T *r, const T *v, T *p, co
 
 // Up to this many partials every block of the kernel that uses a scalar folds them itself
 // (a block and all of them in flight together: 1 to 2 us); above, a kernel of one block does
-// it once.  A solve's iteration at 96x48x6 (27 partials) and 256x128x32 (1024) measured
-// 8 and 6 us less so; at 512x256x64 (8192) each block would read 64 KiB.
+// it once.  Steps of 16 to 1024 partials measured 5 to 16 us less so, of 2048 the same, of 4096
+// up to 2% more and of 8192 (512x256x64, each block would read 64 KiB) 3 to 7% more.
 constexpr int kPBFoldEach = 1024;
 // alpha = rho / (v, r0)
 template <int U>
