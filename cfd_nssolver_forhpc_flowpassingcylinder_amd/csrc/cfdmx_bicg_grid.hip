@@ -47,6 +47,9 @@ namespace cfdmx {
 // a quiet NaN that no arithmetic produces (its payload is set); a partial that is this very
 // value is written as the plain NaN
 constexpr unsigned long long kEmpty = 0x7ff8dead5eed0001ull;
+// looks at a slot before a block gives up (about a microsecond each, of waits that take two or
+// three)
+constexpr int kMaxPolls = 1 << 21;
 constexpr int kGridHalo = 2; // cells of the rows beside the tile that one thread holds
 
 __device__ __forceinline__ void put_through(double *p, double v)
@@ -81,7 +84,7 @@ __global__ void k_grid_slots(int n, unsigned long long *slots, const KState *st,
 template <int PRE, int T, int NC, int PL, bool UNI>
 __global__ void __launch_bounds__(T)
 k_bicg_grid(Geo g, BicgBuffers B, double *__restrict__ x, double *partC,
-            unsigned long long *slots, KState *st, int *failed, int polls, int m0, int count)
+            unsigned long long *slots, KState *st, int *failed, int give_up, int m0, int count)
 {
     static_assert(PL == kChunk || 2 * PL == kChunk, "whole or half march blocks");
     extern __shared__ double lds[];
@@ -112,7 +115,7 @@ k_bicg_grid(Geo g, BicgBuffers B, double *__restrict__ x, double *partC,
     double *Z = lds + PL * WP; // r0, plane by plane
     // slots of phase A (1 sum), B and C (2 sums), by block
     unsigned long long *slotA = slots, *slotB = slots + nb, *slotC = slots + 3 * nb;
-    if (tid == 0) gave_up = 0;
+    if (tid == 0) gave_up = give_up;
     if (tid < PL) {
         cx[0][tid] = tid < len ? g.pa[0].m[i0 + tid] : 0.0;
         cx[1][tid] = tid < len ? g.pa[0].p[i0 + tid] : 0.0;
@@ -264,7 +267,7 @@ k_bicg_grid(Geo g, BicgBuffers B, double *__restrict__ x, double *partC,
             double acc = 0.0;
             if (second) {
                 unsigned long long v = kEmpty;
-                for (int q = 0; q < polls && v == kEmpty; ++q)
+                for (int q = 0; q < kMaxPolls && v == kEmpty; ++q)
                     v = __hip_atomic_load(chain + k * kThreads + w, __ATOMIC_RELAXED,
                                           __HIP_MEMORY_SCOPE_AGENT);
                 if (v == kEmpty) gave_up = 1;
@@ -297,8 +300,7 @@ k_bicg_grid(Geo g, BicgBuffers B, double *__restrict__ x, double *partC,
         if (tid < kThreads) {
             unsigned long long v[2] = {0, 0};
             if (tid < nb) {
-                v[0] = kEmpty;
-                for (int w = 0; w < polls; ++w) {
+                for (int w = 0; w < kMaxPolls; ++w) {
                     v[0] = __hip_atomic_load(slot + ns * tid, __ATOMIC_RELAXED,
                                              __HIP_MEMORY_SCOPE_AGENT);
                     if (ns == 2)
@@ -603,14 +605,14 @@ int bicg_grid_cus(const Geo &g, int pre, int uni, int &cus)
 
 hipError_t launch_bicg_grid(const Geo &g, hipStream_t s, int pre, int uni, BicgBuffers &B,
                             double *x, double *partC, unsigned long long *slots, KState *st,
-                            KState *keep, int *failed, int polls, int m0, int count)
+                            KState *keep, int *failed, int give_up, int m0, int count)
 {
     const int n = bicg_grid_slots(g);
     hipLaunchKernelGGL(k_grid_slots, dim3((n + 255) / 256), dim3(256), 0, s, n, slots,
                        (const KState *)st, m0 == 0 ? keep : nullptr);
     Geo geo = g;
     BicgBuffers buf = B;
-    void *args[] = {&geo, &buf, &x, &partC, &slots, &st, &failed, &polls, &m0, &count};
+    void *args[] = {&geo, &buf, &x, &partC, &slots, &st, &failed, &give_up, &m0, &count};
     return hipLaunchKernel(grid_kernel(g, pre, uni), dim3(grid_blocks_of(g)),
                            dim3(grid_threads(g)), args, grid_lds(g), s);
 }

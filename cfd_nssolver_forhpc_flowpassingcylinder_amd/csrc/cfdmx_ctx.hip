@@ -1459,10 +1459,6 @@ struct SolveTarget {
     KState *kst, *kst_h;
 };
 
-// looks at a partial sum before a block of the resident kernel gives up (about a microsecond
-// each, of waits that take two or three)
-constexpr int kGridPolls = 1 << 21;
-
 static int solve_bicgstab_core(cfdmx_ctx *ctx, const SolveTarget &T, int *iters, double *res)
 {
     hipStream_t s = ctx->stream;
@@ -1487,7 +1483,7 @@ static int solve_bicgstab_core(cfdmx_ctx *ctx, const SolveTarget &T, int *iters,
             PROF(CFDMX_K_BICG_A,
                  e = launch_bicg_grid(g, s, pre, ctx->grid_uni, ctx->B, T.x, ctx->bpart[2],
                                       ctx->grid_slots, T.kst, ctx->grid_keep, ctx->grid_failed,
-                                      give_up ? 0 : kGridPolls, m, kGridBatch));
+                                      give_up, m, kGridBatch));
             if (e == hipSuccess) {
                 HIPCHK(hipMemcpyAsync(T.kst_h, T.kst, sizeof(KState), hipMemcpyDeviceToHost, s));
                 HIPCHK(hipMemcpyAsync(ctx->grid_failed_h, ctx->grid_failed, sizeof(int),

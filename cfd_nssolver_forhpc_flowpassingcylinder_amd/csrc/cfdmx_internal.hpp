@@ -103,11 +103,11 @@ int bicg_grid_slots(const Geo &g);
 // iterations m0 .. m0 + count - 1 in one resident kernel (cfdmx_bicg_grid.hip), on grids for
 // which bicg_grid_cus is not 0.  uni: what bicg_grid_uni says of the grid; partC: 2 * nmarch
 // doubles kept from launch to launch of a solve, slots: bicg_grid_slots values, keep: takes the
-// state the solve starts with (m0 = 0), failed: set to 1 by a block that waited in vain, having
-// looked `polls` times
+// state the solve starts with (m0 = 0), failed: set to 1 by a block that waited in vain, and by
+// all if give_up is 1
 hipError_t launch_bicg_grid(const Geo &g, hipStream_t s, int pre, int uni, BicgBuffers &B,
                             double *x, double *partC, unsigned long long *slots, KState *st,
-                            KState *keep, int *failed, int polls, int m0, int count);
+                            KState *keep, int *failed, int give_up, int m0, int count);
 // Multigrid-preconditioned solve (mixed precision: T = float; the same algorithm in
 // FP64: T = double).  One multigrid level (interior cells, n = (i*ny + j)*nz + k) and
 // the scalars of the preconditioned inner BiCGSTAB.

@@ -25,7 +25,7 @@ static inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 //
 // Bound by memory at the large end: by the counters a pass moves 33 bytes a cell at 512x256x64
 // (25 read, of which 16 are p and the right-hand side and the rest the planes around the tiles;
-// 8 written) where four half sweeps moved 66.  A sweep of a solve of 401, half sweeps and then
+// 8 written) where four half sweeps moved 65.  A sweep of a solve of 401, half sweeps and then
 // passes: 512x256x64 52.9 and 27.1 us (a pass 53, 5.3 TB/s), 420x210x72 48.7 and 24.3, 256x128x128 30.7 and 19.7, 256x128x32 20.9 and
 // 10.8, 64x40x8 12.3 and 6.4, 40x24x4 13.1 and 5.7 us (twelve steps of 0.5 us and a launch).
 // 1024 threads (102 registers): tiles of 32 rows lose a quarter to the halo, of 16 rows a half.

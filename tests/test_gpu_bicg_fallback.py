@@ -1,7 +1,7 @@
 """A resident BiCGSTAB solve that gives up, bit for bit against the oracle: in its first launch,
 and in its second after 1024 iterations have advanced x and the solver's state; then further
-solves, which take launched phases from the start.  Every block's wait ends at once, so the
-kernel ends normally."""
+solves, which take launched phases from the start.  Every block gives up after its first wait,
+so the kernel ends normally."""
 import numpy as np
 import pytest
 
