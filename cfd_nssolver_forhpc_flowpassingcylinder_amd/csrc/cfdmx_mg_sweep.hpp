@@ -245,7 +245,8 @@ template <typename T, int P, bool ZPER> struct MGCol {
 
 // planes that the inputs are loaded ahead: three, or one where a plane's are so many that
 // more would spill registers (P = 4 in float and P = 2 in double at 512x256x64: three
-// planes ahead the up kernel spilled and took 62 and 112 us, one plane ahead 24 and 36 us)
+// planes ahead the up kernel spilled and took 62 and 112 us, one plane ahead 24 and 36 us; what
+// still spills at one plane is in the comment of mg_pairs)
 template <typename T, int P> __host__ __device__ constexpr int mg_ahead()
 {
     return sizeof(T) * P >= 16 ? 1 : 3;
@@ -259,9 +260,9 @@ template <int V> struct MGInt {
 
 // A float dividend below a.tiny gives mg_quot a subnormal part.  A right-hand side of ordinary
 // size has none, so a block divides only in a second pass over its cells, if one of its threads
-// met such a dividend in the first; the results are then written again.  Steps of 24 grids took
-// 0 to 3% longer for looking at the dividends so, 3 to 11% with a branch at every quotient.  In
-// double such a value is 2^-400 times the largest of a residual whose norm does not underflow,
+// met such a dividend in the first; the results are then written again.  Steps of 39 grids took
+// 3% less to 2.5% more with the look at the dividends (nothing in the mean), 3 to 11% more with a
+// branch at every quotient.  In double such a value is 2^-400 times the largest of a residual whose norm does not underflow,
 // and is not looked for.
 template <typename T, class Pass>
 __device__ __forceinline__ void mg_exactly(const MGSweepT<T> &a, Pass &&pass)
