@@ -262,8 +262,8 @@ template <int V> struct MGInt {
 // size has none, so a block divides only in a second pass over its cells, if one of its threads
 // met such a dividend in the first; the results are then written again.  Steps of 39 grids took
 // 3% less to 2.5% more with the look at the dividends (nothing in the mean), 3 to 11% more with a
-// branch at every quotient.  In double such a value is 2^-400 times the largest of a residual whose norm does not underflow,
-// and is not looked for.
+// branch at every quotient.  In double such a value is 2^-400 times the largest of a residual
+// whose norm does not underflow, and is not looked for.
 template <typename T, class Pass>
 __device__ __forceinline__ void mg_exactly(const MGSweepT<T> &a, Pass &&pass)
 {
