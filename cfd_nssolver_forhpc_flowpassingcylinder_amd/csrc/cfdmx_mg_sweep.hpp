@@ -261,20 +261,31 @@ template <int V> struct MGInt {
 // A float dividend below a.tiny gives mg_quot a subnormal part.  A right-hand side of ordinary
 // size has none, so a block divides only in a second pass over its cells, if one of its threads
 // met such a dividend in the first; the results are then written again.  Steps of 39 grids took
-// 3% less to 2.5% more with the look at the dividends (nothing in the mean), 3 to 11% more with a
+// 4% less to 3% more with the look at the dividends (nothing in the mean), 3 to 11% more with a
 // branch at every quotient.  In double such a value is 2^-400 times the largest of a residual
 // whose norm does not underflow, and is not looked for.
-template <typename T, class Pass>
-__device__ __forceinline__ void mg_exactly(const MGSweepT<T> &a, Pass &&pass)
+template <typename T, class Pass> __device__ __forceinline__ void mg_exactly(Pass &&pass)
 {
-    const unsigned least = pass(std::false_type());
-    if constexpr (std::is_same<T, float>::value)
-        if (__syncthreads_or(least < 2u * __float_as_uint(a.tiny) - 1u)) pass(std::true_type());
+    if (!pass(std::false_type())) return;
+    __syncthreads(); // the flag has been read
+    pass(std::true_type());
+}
+// whether a thread of the block met a small dividend.  flag: an entry of LDS that the last step
+// of a pass, which no barrier follows, neither reads nor writes; its zero is the zero behind a
+// row.  (Four bytes of LDS of its own took a CU's second block from the largest tiles: a step of
+// 1024x512x128 cells 21.4 -> 28.0 ms.)
+template <typename T, bool EXACT>
+__device__ __forceinline__ bool mg_small(const MGSweepT<T> &a, unsigned least, T *flag)
+{
+    if constexpr (EXACT || !std::is_same<T, float>::value) return false;
+    if (least < 2u * __float_as_uint((float)a.tiny) - 1u) *flag = (T)1;
+    __syncthreads();
+    return *flag != (T)0;
 }
 
 // GEN: 0 = z-only coarsening (fx = fy = 1, fz = 2); 1 = any other, by the factors in a
 template <typename T, int P, bool ZPER, int GEN, bool EXACT>
-__device__ __forceinline__ unsigned mg_down(const MGSweepT<T> &a, const MGCol<T, P, ZPER> &c)
+__device__ __forceinline__ bool mg_down(const MGSweepT<T> &a, const MGCol<T, P, ZPER> &c)
 {
     extern __shared__ double mg_lds[];
     unsigned least = ~0u;
@@ -438,40 +449,44 @@ __device__ __forceinline__ unsigned mg_down(const MGSweepT<T> &a, const MGCol<T,
             b2m[q] = b2[q];
             rb[q] = rbn[q];
         }
-        __syncthreads();
     };
     auto march = [&](auto PAR_) MG_INLINE {
         constexpr int A = decltype(PAR_)::v;
         for (int t = 0;;) {
             step(MGInt<0>(), MGInt<A>(), first + t);
             if (++t >= steps) break;
+            __syncthreads();
             step(MGInt<1>(), MGInt<1 - A>(), first + t);
             if (++t >= steps) break;
+            __syncthreads();
             step(MGInt<2>(), MGInt<A>(), first + t);
             if (++t >= steps) break;
+            __syncthreads();
             step(MGInt<3>(), MGInt<1 - A>(), first + t);
             if (++t >= steps) break;
+            __syncthreads();
         }
     };
     // a wave's parity is one value, and every wave takes the same number of steps (and so
     // of barriers) on either side
     if (__builtin_amdgcn_readfirstlane(c.par0)) march(MGInt<1>());
     else march(MGInt<0>());
-    return least;
+    // the slot of L1 that the last step writes is read by none
+    return mg_small<T, EXACT>(a, least, L1 + ((steps - 1) & 1) * SL + a.pairs);
 }
 template <typename T, int P, bool ZPER, int GEN>
 __global__ void __launch_bounds__(kMGSweepThreads) k_mg_down(MGSweepT<T> a)
 {
     MGCol<T, P, ZPER> c;
     if (!c.init(a)) return;
-    mg_exactly(a, [&](auto exact) {
+    mg_exactly<T>([&](auto exact) {
         return mg_down<T, P, ZPER, GEN, decltype(exact)::value>(a, c);
     });
 }
 
 // FZ2: the level was coarsened in z (a pair's cells have one parent)
 template <typename T, int P, bool ZPER, bool FZ2, bool EXACT>
-__device__ __forceinline__ unsigned mg_up(const MGSweepT<T> &a, const MGCol<T, P, ZPER> &c)
+__device__ __forceinline__ bool mg_up(const MGSweepT<T> &a, const MGCol<T, P, ZPER> &c)
 {
     extern __shared__ double mg_lds[];
     unsigned least = ~0u;
@@ -570,32 +585,36 @@ __device__ __forceinline__ unsigned mg_up(const MGSweepT<T> &a, const MGCol<T, P
             xr2[o][q] = x3[q];
             r2m[q] = r2[q];
         }
-        __syncthreads();
     };
     auto march = [&](auto PAR_) MG_INLINE {
         constexpr int A = decltype(PAR_)::v;
         for (int t = 0;;) {
             step(MGInt<0>(), MGInt<A>(), first + t);
             if (++t >= steps) break;
+            __syncthreads();
             step(MGInt<1>(), MGInt<1 - A>(), first + t);
             if (++t >= steps) break;
+            __syncthreads();
             step(MGInt<2>(), MGInt<A>(), first + t);
             if (++t >= steps) break;
+            __syncthreads();
             step(MGInt<3>(), MGInt<1 - A>(), first + t);
             if (++t >= steps) break;
+            __syncthreads();
         }
     };
     // as in mg_down; plane i's black cells have the other parity
     if (__builtin_amdgcn_readfirstlane(c.par0)) march(MGInt<0>());
     else march(MGInt<1>());
-    return least;
+    // the slot of L1 that the last step writes is read by none
+    return mg_small<T, EXACT>(a, least, L1 + ((steps - 1) & 1) * SL + a.pairs);
 }
 template <typename T, int P, bool ZPER, bool FZ2>
 __global__ void __launch_bounds__(kMGSweepThreads) k_mg_up(MGSweepT<T> a)
 {
     MGCol<T, P, ZPER> c;
     if (!c.init(a)) return;
-    mg_exactly(a, [&](auto exact) {
+    mg_exactly<T>([&](auto exact) {
         return mg_up<T, P, ZPER, FZ2, decltype(exact)::value>(a, c);
     });
 }
